@@ -116,7 +116,8 @@ typedef struct PpmBatchParams {
     int cap;            /* |E|>100 rescale of the grid */
     int nz;             /* z-steps of every scan */
     int nmol, nitems;
-    int vz;             /* grid voxels per thread along z: 4 or 8 */
+    int vz;             /* size of a grid tile: 4 (small) or 8 (large); voxels per thread along z of a
+                           directly summed grid */
     int tile_w;         /* pixels along iy of a wavefront's pixel tile: 4, 8 or 16 (64/tile_w along ix) */
     int mode;           /* PPM_BATCH_FUSED, PPM_BATCH_GRID_ONLY or PPM_BATCH_RELAX_ONLY */
     int df_taps, df_nz_out;
@@ -491,6 +492,12 @@ int ppm_direct_morse_vjp(const float* atoms, const float* cMs, int na,
 
 /* Bytes of device workspace (work queue, per-molecule counters and flags) of a batch of nmol. */
 size_t ppm_batch_workspace_size(int nmol);
+
+/* Number of grid tiles a molecule divides into at params->vz (params: model, vz, Qs, QZs; the rest is
+ * not read): the n_grid_items with which every work queue item is one workgroup's share.  Fewer or
+ * more items give the same grid (an item takes the tiles item, item + n_grid_items, ...).  Host
+ * pointers; -1 on invalid arguments. */
+int ppm_batch_grid_items(const PpmMolDesc* mol, const PpmBatchParams* params);
 
 /* Batched forward (no reference counterpart: the reference runs one image at a time through
  * make_forcefield / run_scan / compute_df, spammm/SPM/AFM.py:897-1010, :3048-3089).

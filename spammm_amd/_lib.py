@@ -58,7 +58,7 @@ EXPORTS = (
     "ppm_ewald_cluster", "ppm_ewald_grid_workspace_size", "ppm_ewald_tip_grid", "ppm_ewald_kept_count_offset",
     "ppm_relax_state_diag", "ppm_relax_strokes_2d", "ppm_grid_project_window", "ppm_relax_strokes_tilted_window",
     "ppm_batch_forward_noalloc", "ppm_fdbm_release_plans", "ppm_relax_strokes_tilted_df", "ppm_stream_create",
-    "ppm_stream_destroy",
+    "ppm_stream_destroy", "ppm_batch_grid_items",
 )
 
 _lib = None
@@ -163,6 +163,8 @@ def load():
     L.ppm_relax_state_diag.argtypes = [vp, P(PpmGridSpec), vp, i, i, P(PpmTip), vp, vp, vp]
     L.ppm_batch_workspace_size.restype = ctypes.c_size_t
     L.ppm_batch_workspace_size.argtypes = [i]
+    L.ppm_batch_grid_items.restype = i
+    L.ppm_batch_grid_items.argtypes = [vp, vp]
     L.ppm_batch_forward.restype = i
     L.ppm_batch_forward.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, ctypes.c_size_t, i, i, vp]
     L.ppm_relax_strokes_tilted_df.restype = i

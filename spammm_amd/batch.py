@@ -49,7 +49,7 @@ MODES = {"fused": 0, "grid_only": 1, "relax_only": 2}
 
 @dataclass
 class LaunchConfig:
-    vz: int = 8                 # grid voxels per thread along z
+    vz: int = 8                 # grid tile size (8 large, 4 small)
     tile_w: int = 8             # pixels along iy of a wavefront's 64-pixel tile
     workers_per_cu: int = 3     # persistent workgroups per compute unit
     schedule: str = "fused"     # "fused" (one launch) or "two_phase" (grid launch, then relax launch)
@@ -138,9 +138,7 @@ class BatchForward:
             d.npbc_a, d.npbc_b = int(w.npbc[0]), int(w.npbc[1])
             d.pix_off, d.scan_nx, d.scan_ny = pix_off, int(w.nxy[0]), int(w.nxy[1])
             d.item_off = item_off
-            vz_max = 4   # grid items are counted for the smallest vz so every launch shape fits
-            d.n_grid_items = ((nx * ny + 255) // 256) * ((nzw + vz_max - 1) // vz_max)
-            d.n_relax_items = 0          # set per launch shape in _set_items
+            d.n_grid_items = d.n_relax_items = 0          # set per launch shape in _set_items
             d.grid_off = grid_off
             d.p0, d.dA, d.dB, d.dC = (_lib.f4(v) for v in (sp.p0, sp.dA, sp.dB, sp.dC))
             d.dinvA, d.dinvB, d.dinvC = (_lib.f4(v) for v in (sp.dinvA, sp.dinvB, sp.dinvC))
@@ -200,8 +198,11 @@ class BatchForward:
         if cfg.lag < 0:
             raise ValueError("lag must be >= 0")
         th = 64 // cfg.tile_w
+        L, P = _lib.load(), self._params(cfg, MODES["fused"], 0)
         for d in self.descs_host:
-            d.n_grid_items = ((d.nx * d.ny + 255) // 256) * ((d.nzw + cfg.vz - 1) // cfg.vz)
+            d.n_grid_items = L.ppm_batch_grid_items(ctypes.addressof(d), ctypes.addressof(P))
+            if d.n_grid_items < 1:
+                raise ValueError(f"ppm_batch_grid_items: {L.ppm_last_error().decode()}")
             tiles = ((d.scan_nx + th - 1) // th) * ((d.scan_ny + cfg.tile_w - 1) // cfg.tile_w)
             d.n_relax_items = (tiles + 3) // 4
         n = len(self.descs_host)
@@ -227,10 +228,10 @@ class BatchForward:
         self.descs_dev.copy_(torch.as_tensor(raw.copy()))
         self._items_for = key
 
-    def _params(self, cfg: LaunchConfig, mode: int) -> PpmBatchParams:
+    def _params(self, cfg: LaunchConfig, mode: int, nitems=None) -> PpmBatchParams:
         P = PpmBatchParams()
         P.model, P.cap, P.nz = self.model, int(self.cap), self.nz
-        P.nmol, P.nitems = len(self.molecules), self.nitems
+        P.nmol, P.nitems = len(self.molecules), self.nitems if nitems is None else nitems
         P.vz, P.tile_w, P.mode = cfg.vz, cfg.tile_w, mode
         if self.dfop is not None:
             P.df_taps, P.df_nz_out = self.dfop.taps, self.dfop.n_out

@@ -601,6 +601,16 @@ int ppm_direct_morse_vjp(const float* atoms, const float* cMs, int na, const flo
                              grad, (hipStream_t)stream);
 }
 
+int ppm_batch_grid_items(const PpmMolDesc* mol, const PpmBatchParams* params) {
+    g_err[0] = 0;
+    if (!mol || !params || mol->na < 0 || mol->nx < 1 || mol->ny < 1 || mol->nz < 1 || mol->nzw < 1 || mol->klo < 0 ||
+        mol->npbc_a < 0 || mol->npbc_b < 0 || (params->vz != 4 && params->vz != 8)) {
+        set_error("ppm_batch_grid_items: invalid argument");
+        return -1;
+    }
+    return batch_grid_items(*mol, *params);
+}
+
 size_t ppm_batch_workspace_size(int nmol) { return nmol < 1 ? 0 : batch_workspace(nmol); }
 
 static int check_batch(const char* fn, const PpmMolDesc* mols, const PpmBatchParams* params, const float* atoms,

@@ -20,6 +20,7 @@
 #include <mutex>
 
 #include "ppm_grid_core.hpp"
+#include "ppm_grid_far.hpp"
 #include "ppm_relax_core.hpp"
 
 namespace ppm {
@@ -55,7 +56,7 @@ __global__ void k_batch_status(Queue* q, int nmol, int* __restrict__ status) {
     if (i < nmol) status[1 + i] = q_flag(q, nmol)[i];
 }
 
-__device__ GridArgs mol_grid_args(const PpmMolDesc& d, const PpmBatchParams& P) {
+__host__ __device__ inline GridArgs mol_grid_args(const PpmMolDesc& d, const PpmBatchParams& P) {
     GridArgs a{};
     a.nx = d.nx; a.ny = d.ny; a.nz = d.nz; a.ncol = d.nx * d.ny;
     for (int k = 0; k < 3; ++k) {
@@ -101,16 +102,62 @@ __device__ rc::TiltArgs tilt_args(const PpmBatchParams& P) {
     return t;
 }
 
+// Grid work of a molecule in units one workgroup takes: the direct sum's tiles of 256 columns x V
+// planes, or (interpolated grids, ppm_grid_far.hpp) blocks of 16^3 voxels or shares of 32^3: V = 8
+// halves them, V = 4 takes a quarter at a time.
+struct GridUnits {
+    int level, nx, ny, nz, split;      // level 0: nx column blocks (ny = 1)
+    __host__ __device__ int count() const { return nx * ny * nz * split; }
+};
+
+__host__ __device__ inline GridUnits grid_units(const GridArgs& a, int model, int V, int klo, int nzw) {
+    GridUnits u;
+    u.level = gf::far_level(a, model);
+    if (u.level == 0) {
+        u.nx = (a.ncol + 255) / 256;
+        u.ny = 1;
+        u.nz = (nzw + V - 1) / V;
+        u.split = 1;
+    } else {
+        const int B = u.level == 2 ? 2 * gf::kB : gf::kB;
+        u.nx = (a.nx + B - 1) / B;
+        u.ny = (a.ny + B - 1) / B;
+        u.nz = (klo + nzw - 1) / B - klo / B + 1;
+        u.split = u.level == 2 ? (V == 8 ? 2 : 4) : 1;
+    }
+    return u;
+}
+
+union GridShared {
+    Site sites[gc::kTile + 1];
+    gf::Shared far;
+};
+
+// Grid item `local` of the molecule's d.n_grid_items: its units local, local + n_grid_items, ...
 template <int MODEL, bool HASQ0, int V, bool OFFQ>
 __device__ void do_grid_item(const PpmMolDesc& d, const PpmBatchParams& P, int local, const float4* atoms,
-                             const float* cpar, float4* grids, Site* sites) {
+                             const float* cpar, float4* grids, GridShared& sh) {
     const GridArgs a = mol_grid_args(d, P);
-    const int ncolblk = (a.ncol + 255) / 256;
-    const int cb = local % ncolblk, zb = local / ncolblk;
-    const int cs = MODEL == PPM_MODEL_LJ ? 2 : 4;
-    gc::grid_tile<MODEL, HASQ0, V, true, OFFQ ? gc::kOffStatic : gc::kOffNone>(atoms + d.atom_off, cpar + (size_t)d.atom_off * cs, a, sites,
-                                         cb * 256 + threadIdx.x, d.klo + zb * V, d.klo + d.nzw, grids + d.grid_off,
-                                         d.klo);
+    const GridUnits n = grid_units(a, MODEL, V, d.klo, d.nzw);
+    constexpr int OFF = OFFQ ? gc::kOffStatic : gc::kOffNone;
+    const int cs = MODEL == PPM_MODEL_LJ ? 2 : 4, kend = d.klo + d.nzw;
+    const float4* at = atoms + d.atom_off;
+    const float* cp = cpar + (size_t)d.atom_off * cs;
+    float4* out = grids + d.grid_off;
+    for (int u = local; u < n.count(); u += d.n_grid_items) {
+        const int x = u % n.nx, y = u / n.nx % n.ny, r = u / (n.nx * n.ny), z = r % n.nz, part = r / n.nz;
+        __syncthreads();               // the shared buffers of the previous unit are free
+        if (n.level == 0)
+            gc::grid_tile<MODEL, HASQ0, V, true, OFF>(at, cp, a, sh.sites, x * 256 + threadIdx.x, d.klo + z * V, kend,
+                                                      out, d.klo);
+        else if (MODEL == PPM_MODEL_LJ && n.level == 2)
+            gf::far_blocks<MODEL, HASQ0, OFF, true, float>(sh.far, at, cp, a, x * 32, y * 32, (d.klo / 32 + z) * 32,
+                                                           part * 8 / n.split, (part + 1) * 8 / n.split, d.klo, kend,
+                                                           out, nullptr);
+        else
+            gf::far_blocks<MODEL, HASQ0, OFF, false, float>(sh.far, at, cp, a, x * 16, y * 16, (d.klo / 16 + z) * 16, 0,
+                                                            1, d.klo, kend, out, nullptr);
+    }
 }
 
 __device__ void do_relax_item(const PpmMolDesc& d, const PpmBatchParams& P, int local, const float4* grids,
@@ -144,15 +191,16 @@ __device__ void do_relax_item(const PpmMolDesc& d, const PpmBatchParams& P, int 
         rc::relax_tilted_lane<false, false>(g, start, t, FEs + o, pp, df ? &dfo : nullptr, dr);
 }
 
-// OFFQ: the tip has charge sites at a nonzero z offset (compiled out when it has none).
-template <int MODEL, bool HASQ0, int V, bool OFFQ>
-__global__ __launch_bounds__(256) void k_batch(const PpmMolDesc* __restrict__ mols, PpmBatchParams P,
+// OFFQ: the tip has charge sites at a nonzero z offset (compiled out when it has none).  GRID = false:
+// a launch of relaxation blocks only, without the grid code's registers and LDS (53 KB: 3 workgroups per
+// compute unit), which leaves the relaxation more waves.
+template <int MODEL, bool HASQ0, int V, bool OFFQ, bool GRID>
+__global__ __launch_bounds__(256, GRID ? 3 : 4) void k_batch(const PpmMolDesc* __restrict__ mols, PpmBatchParams P,
                                                const float4* __restrict__ atoms, const float* __restrict__ cpar,
                                                float4* __restrict__ grids, float4* __restrict__ FEs,
                                                float4* __restrict__ PPs, float* __restrict__ df,
                                                const float* __restrict__ dfW, const int* __restrict__ dfStart,
                                                Queue* q) {
-    __shared__ Site sites[gc::kTile + 1];
     __shared__ int s_item, s_mol, s_local;
     int* done = q_done(q);
     int* flags = q_flag(q, P.nmol);
@@ -199,8 +247,9 @@ __global__ __launch_bounds__(256) void k_batch(const PpmMolDesc* __restrict__ mo
         const PpmMolDesc& d = mols[m];
         signal_m = -1;
         if (local < d.n_grid_items) {
-            if (P.mode != PPM_BATCH_RELAX_ONLY) {
-                do_grid_item<MODEL, HASQ0, V, OFFQ>(d, P, local, atoms, cpar, grids, sites);
+            if constexpr (GRID) {
+                __shared__ GridShared sh;
+                do_grid_item<MODEL, HASQ0, V, OFFQ>(d, P, local, atoms, cpar, grids, sh);
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
                 __syncthreads();            // every thread's tile stores precede the signal
                 signal_m = m;
@@ -229,10 +278,10 @@ void launch_v(int V, dim3 grd, hipStream_t st, const PpmMolDesc* mols, const Ppm
               const float* cpar, float4* grids, float4* FEs, float4* PPs, float* df, const float* dfW,
               const int* dfStart, Queue* q) {
     if (V == 8)
-        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 8, OFFQ>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
+        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 8, OFFQ, true>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
                            PPs, df, dfW, dfStart, q);
     else
-        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 4, OFFQ>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
+        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 4, OFFQ, true>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
                            PPs, df, dfW, dfStart, q);
 }
 
@@ -250,6 +299,10 @@ void launch_q(bool hasq0, bool offq, int V, dim3 grd, hipStream_t st, const PpmM
 }
 
 }  // namespace
+
+int batch_grid_items(const PpmMolDesc& d, const PpmBatchParams& P) {
+    return grid_units(mol_grid_args(d, P), P.model, P.vz, d.klo, d.nzw).count();
+}
 
 size_t batch_workspace(int nmol) { return sizeof(Queue) + 2 * (size_t)nmol * sizeof(int); }
 
@@ -306,7 +359,10 @@ int launch_batch(const PpmMolDesc* mols, const PpmBatchParams& P, const float* a
     float4* gr = reinterpret_cast<float4*>(grids);
     float4* fe = reinterpret_cast<float4*>(FEs);
     float4* pp = reinterpret_cast<float4*>(PPs);
-    if (P.model == PPM_MODEL_LJ)
+    if (P.mode == PPM_BATCH_RELAX_ONLY)      // no pair law takes part
+        hipLaunchKernelGGL((k_batch<PPM_MODEL_LJ, false, 8, false, false>), grd, dim3(256), 0, stream, mols, P, at, cpar,
+                           gr, fe, pp, df, dfW, dfStart, q);
+    else if (P.model == PPM_MODEL_LJ)
         launch_q<PPM_MODEL_LJ>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, fe, pp, df, dfW, dfStart, q);
     else
         launch_q<PPM_MODEL_MORSE>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, fe, pp, df, dfW, dfStart, q);

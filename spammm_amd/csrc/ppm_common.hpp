@@ -93,6 +93,7 @@ int launch_ewald_cluster(const float* pts, int np, const float* ions, int ni, fl
 int launch_ewald_tip_grid(const void* system, int n_layers, int n_harm, const double a[2], const double b[2],
                           const PpmGridSpec& gs, const float Qs[4], const float QZs[4], int accumulate,
                           void* workspace, float* grid, hipStream_t stream);
+int batch_grid_items(const PpmMolDesc& d, const PpmBatchParams& P);
 size_t batch_workspace(int nmol);
 // Largest batch of the allocation-free batch entry point (its file-scope scratch holds the queue,
 // counters and flags of this many molecules: 512 KiB + 16 B per GPU).

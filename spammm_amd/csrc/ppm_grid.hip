@@ -9,9 +9,12 @@
 //   cap    |E|>100 => all four channels scaled by 100/|E|   kernels/AFM.cl:984-985
 //   images atom shifted by ix*lvA + iy*lvB, ix,iy in [-npbc,npbc] (kernels/gridFF.cl:960-996)
 //
-// Design (FP32 VALU-bound):
+// Two forms, chosen by far_level from the grid alone.  Grids of more than a few sites and blocks
+// take the interpolated one (ppm_grid_far.hpp): the flake's 300x300x240 voxels x 1800 sites 13.06 -> 0.73 ms,
+// a 9216-site slab on 320x320x96 at 0.05 A 32.9 -> 1.07 ms.  The rest is the direct sum (FP32 VALU-bound):
 //   * one workgroup = 256 columns (ia,ib) x V consecutive z voxels per thread (V = 16 or 8
-//     for LJ, chosen per launch shape; 8 for Morse, 4 for a tilted dC); voxels of one thread
+//     for LJ, chosen per launch shape; 8 for Morse, 4 for a tilted dC, 1 for launches of few
+//     workgroups); voxels of one thread
 //     share dx, dy and dx^2+dy^2 for every site;
 //   * the atom x image "sites" are expanded once per 256-site tile into LDS by the
 //     workgroup (one site per thread), then read as broadcasts by every lane;
@@ -21,11 +24,15 @@
 #include <algorithm>
 
 #include "ppm_grid_core.hpp"
+#include "ppm_grid_far.hpp"
 
 namespace ppm {
 namespace {
 
 using namespace gc;
+using gf::expected_near;
+using gf::far_level;
+using gf::near2;
 
 // Planes [klo, kend) of the grid (klo = 0, kend = nz: the whole grid), stored from plane klo on:
 // a z window has the voxel values of the same planes of the whole grid, bit for bit.
@@ -37,6 +44,21 @@ __global__ __launch_bounds__(256) void k_grid_project(const float4* __restrict__
     __shared__ Site sites[kTile + 1];
     grid_tile<MODEL, HASQ0, V, DCZ, kOffDynamic, ACC>(atoms, cpar, a, sites, blockIdx.x * 256 + threadIdx.x,
                                                       klo + blockIdx.y * V, kend, out, klo, base);
+}
+
+// The interpolated form: workgroup (blockIdx.x, blockIdx.y) takes the (x,y) and z block (two levels: of
+// 32 voxels a side, one level: 16) of the planes [klo, kend); blocks are aligned to plane 0.
+template <int MODEL, bool HASQ0, bool OFFS, bool TWO, typename ACC>
+__global__ __launch_bounds__(256, sizeof(ACC) == 8 ? 1 : TWO ? 2 : 3) void k_grid_far(
+    const float4* __restrict__ atoms, const float* __restrict__ cpar, GridArgs a, float4* __restrict__ out,
+    const float4* base, int klo, int kend, int split) {
+    __shared__ gf::Shared s;
+    constexpr int B = TWO ? 2 * gf::kB : gf::kB;
+    const int nbx = (a.nx + B - 1) / B;
+    const int by = (int)blockIdx.x / nbx, bx = (int)blockIdx.x - by * nbx;
+    gf::far_blocks<MODEL, HASQ0, OFFS ? kOffDynamic : kOffNone, TWO, ACC>(
+        s, atoms, cpar, a, bx * B, by * B, (klo / B + (int)blockIdx.y) * B, (int)blockIdx.z * (TWO ? 8 : 1) / split,
+        ((int)blockIdx.z + 1) * (TWO ? 8 : 1) / split, klo, kend, out, base);
 }
 
 // ── grid -> atom adjoint ─────────────────────────────────────────────────────────────
@@ -402,12 +424,49 @@ bool lj_16_voxels(int ncol, int nzw) {
     return 610 * k16 + 290 + (k16 == 1 ? 120 : 0) <= 334 * k8 + 180;
 }
 
+// Workgroups per 2^3 blocks of the two-level form (1, 2, 4 or 8; each repeats the sums at the 32^3
+// voxels' nodes and takes its share of the blocks; the bits do not depend on it).  With F = 512 x far
+// sites, S the work of the 8 blocks (in pair evaluations) and nb launched 2^3 blocks, the time
+// measured over 98..1125 blocks and 180..9216 sites follows nb (s F + S) / 2.9e9 + 0.6 (F + S / s) /
+// 3.5e6 ms: the card's rate and one workgroup's serial time.  300x300x62 planes, 1800 sites: s = 1, 2,
+// 4, 8 take 597, 459, 522, 714 us; 300x300x240: 722, 916, 1324, 2247.
+int far_split(const GridArgs& a, double nb) {
+    const double n = a.nsites, near = expected_near(a, near2(a, false)), mid = expected_near(a, near2(a, true));
+    const double F = 512.0 * (n - mid), S = 8.0 * (512.0 * (mid - near) + 4096.0 * near + 62e3);
+    int best = 1;
+    double t = 0.0;
+    for (int s = 1; s <= 8; s *= 2) {
+        const double ts = nb * (s * F + S) / 2.9e9 + 0.6 * (F + S / s) / 3.5e6;
+        if (s == 1 || ts < t) { best = s; t = ts; }
+    }
+    return best;
+}
+
+template <int MODEL, bool HASQ0, bool TWO>
+int launch_far(const float4* atoms, const float* cpar, const GridArgs& a, float4* out, const float4* base, bool acc64,
+               hipStream_t st, int klo, int kend) {
+    constexpr int B = TWO ? 2 * gf::kB : gf::kB;
+    const unsigned nxy = (unsigned)(((a.nx + B - 1) / B) * ((a.ny + B - 1) / B)), nz = (kend - 1) / B - klo / B + 1;
+    const int split = TWO ? far_split(a, (double)nxy * nz) : 1;
+    const dim3 grd(nxy, nz, (unsigned)split), blk(256);
+#define PPM_FAR(OF, AC) \
+    hipLaunchKernelGGL((k_grid_far<MODEL, HASQ0, OF, TWO, AC>), grd, blk, 0, st, atoms, cpar, a, out, base, klo, kend, split)
+    if (acc64) { if (a.noff) PPM_FAR(true, double); else PPM_FAR(false, double); }
+    else { if (a.noff) PPM_FAR(true, float); else PPM_FAR(false, float); }
+#undef PPM_FAR
+    return check_launch("grid_project_far");
+}
+
 template <int MODEL, bool HASQ0>
 int dispatch(const float4* atoms, const float* cpar, const GridArgs& a, float4* out, const float4* base,
              bool acc64, hipStream_t st, int klo, int nzw) {
     const bool dcz = (a.dC[0] == 0.f && a.dC[1] == 0.f);
     const int kend = klo + nzw;
     dim3 blk(256);
+    const int level = far_level(a, MODEL);
+    if constexpr (MODEL == PPM_MODEL_LJ)
+        if (level == 2) return launch_far<MODEL, HASQ0, true>(atoms, cpar, a, out, base, acc64, st, klo, kend);
+    if (level) return launch_far<MODEL, HASQ0, false>(atoms, cpar, a, out, base, acc64, st, klo, kend);
     if (acc64) {          // FP64 sums: 8 voxels per thread (16 would need 128 VGPRs of sums alone)
         const int V = dcz ? 8 : 4;
         dim3 grd((a.ncol + 255) / 256, (nzw + V - 1) / V);
@@ -420,7 +479,15 @@ int dispatch(const float4* atoms, const float* cpar, const GridArgs& a, float4* 
         return check_launch("grid_project_acc64");
     }
     if (dcz) {
-        if (MODEL == PPM_MODEL_LJ && nzw >= 16 && lj_16_voxels(a.ncol, nzw)) {   // 16 on Morse: +2 %
+        // few workgroups of 8 voxels per thread (up to ~4 per compute unit): one voxel per thread, so the
+        // sites' serial loop has more waves to hide it (same bits).  8 against 1, microseconds: 48x48x40
+        // voxels and 180 sites 57 / 19, 104x104x60 and 540 246 / 165, 170x170x60 and 1800 1430 / 1260;
+        // past that 8 wins: 177x177x150 and 180 338 / 341, 160^3 and 180 275 / 295
+        if ((long long)((a.ncol + 255) / 256) * ((nzw + 7) / 8) <= 4LL * device_cus()) {
+            dim3 grd((a.ncol + 255) / 256, nzw);
+            hipLaunchKernelGGL((k_grid_project<MODEL, HASQ0, 1, true>), grd, blk, 0, st, atoms, cpar, a, out, base, klo,
+                               kend);
+        } else if (MODEL == PPM_MODEL_LJ && nzw >= 16 && lj_16_voxels(a.ncol, nzw)) {   // 16 on Morse: +2 %
             dim3 grd((a.ncol + 255) / 256, (nzw + 15) / 16);
             hipLaunchKernelGGL((k_grid_project<MODEL, HASQ0, 16, true>), grd, blk, 0, st, atoms, cpar, a, out, base,
                                klo, kend);

@@ -1,0 +1,593 @@
+// ppm_grid_far.hpp — force-field grid projection with interpolated far fields (device code shared
+// by the plain and the batched kernels).
+//
+// The direct sum (ppm_grid_core.hpp) evaluates every atom image at every voxel and is bound by the
+// VALU: 1800 sites per voxel on a 300x300x240 grid, while the field of a site a few block sizes
+// away is a smooth function over a block of voxels.  Here a block's voxels are split from its sites
+// by distance:
+//   * near sites are summed directly at the 16^3 voxels of a block;
+//   * the other sites are summed at 8^3 Chebyshev nodes of the block (512 points instead of 4096),
+//     and the polynomial through the node values is evaluated at the voxels;
+//   * with two levels a workgroup takes 2^3 blocks: sites far from all of them are summed at the
+//     8^3 nodes of the 32^3 voxels (512 instead of 32768), and that polynomial is evaluated at the
+//     nodes of each block.
+// No site is left out: every site enters every voxel once, through exactly one of the three sums.
+// The interpolation error of a site at distance d from the centre of a block of half-width h falls
+// as (d/h + sqrt((d/h)^2 - 1))^-8; kRatio h is where it passes below the FP32 rounding of the sums.
+// Blocks are aligned to voxel 0 of the grid, whatever planes are stored, and which sums a site takes
+// depends on the block alone, so a z window has the bits of the same planes of the whole grid.
+//
+// Node positions are taken relative to the block's centre (the centre in FP64), which leaves less
+// rounding in dx, dy, dz than absolute FP32 positions.
+#pragma once
+#pragma clang fp contract(off)
+#include "ppm_grid_core.hpp"
+
+namespace ppm {
+namespace gf {
+
+using gc::GridArgs;
+using gc::Site;
+
+constexpr int kM = 8;              // Chebyshev nodes per axis
+constexpr int kB = 16;             // voxels per axis of a block
+constexpr int kList = 512;         // sites near a workgroup's blocks that LDS holds at a time
+constexpr float kRatio = 10.0f;       // near: closer than kRatio half-widths
+constexpr int kMinMid = 6;         // fewer sites than this are cheaper summed at the voxels
+
+// cos((2 i + 1) pi / 16): the nodes on [-1, 1], descending
+constexpr double kNode[kM] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
+                              0.19509032201612826785, -0.19509032201612826785, -0.55557023301960222474,
+                              -0.83146961230254523708, -0.98078528040323044913};
+
+// Weight of node k in the polynomial through the 8 nodes, at u.
+constexpr double lagrange(int k, double u) {
+    double w = 1.0;
+    for (int j = 0; j < kM; ++j)
+        if (j != k) w *= (u - kNode[j]) / (kNode[k] - kNode[j]);
+    return w;
+}
+
+struct Tables {
+    float vox[kB][kM];        // block nodes -> the 16 voxels of an axis
+    float sub[2][kM][kM];     // nodes of 32 voxels -> the nodes of their lower / upper 16
+    constexpr Tables() : vox(), sub() {
+        for (int k = 0; k < kM; ++k) {
+            for (int i = 0; i < kB; ++i) vox[i][k] = (float)lagrange(k, (i - 7.5) / 7.5);
+            for (int h = 0; h < 2; ++h)
+                for (int i = 0; i < kM; ++i) sub[h][i][k] = (float)lagrange(k, ((h ? 8.0 : -8.0) + 7.5 * kNode[i]) / 15.5);
+        }
+    }
+};
+constexpr Tables kTab{};
+static __constant__ Tables c_tab = kTab;
+
+struct Shared {
+    float top[4][kM * kM * kM];                // node values of the 32^3 voxels, per channel
+    Site list[kList];
+    unsigned short mid[kList], near[kList];    // entries of list summed at the nodes / at the voxels
+    float a[4][kM * 72];                       // node values of a block; its z-interpolated planes
+    union {
+        float b[4][kM * 136];
+        Site tile[256];
+    };
+    int cnt[2][4];
+};
+
+// Largest squared half edge of a voxel-step cube, in units of half voxels: a skewed or flat block
+// counts with its largest edge or diagonal / sqrt(3).
+__host__ __device__ inline double step2(const GridArgs& a) {
+    double m = 0.0, e[3] = {0.0, 0.0, 0.0};
+    for (int s = 0; s < 4; ++s) {
+        const double sb = (s & 1) ? -1.0 : 1.0, sc = (s & 2) ? -1.0 : 1.0;
+        double d = 0.0;
+        for (int q = 0; q < 3; ++q) {
+            const double v = (double)a.dA[q] + sb * (double)a.dB[q] + sc * (double)a.dC[q];
+            d += v * v;
+        }
+        if (d / 3.0 > m) m = d / 3.0;
+    }
+    for (int q = 0; q < 3; ++q) {
+        e[0] += (double)a.dA[q] * (double)a.dA[q];
+        e[1] += (double)a.dB[q] * (double)a.dB[q];
+        e[2] += (double)a.dC[q] * (double)a.dC[q];
+    }
+    for (int q = 0; q < 3; ++q)
+        if (e[q] > m) m = e[q];
+    return m;
+}
+
+// Squared near radii: kRatio half-widths of a block, and of 2^3 blocks.
+__host__ __device__ inline double near2(const GridArgs& a, bool top) {
+    const double h = (top ? kB - 0.5 : 0.5 * (kB - 1)) * (double)kRatio;
+    return step2(a) * (h * h);
+}
+
+// Expected number of sites within r of a point of the molecule's plane, from the sites' area density
+// (over the lattice cell of the images, or over the grid), averaged over heights within r.
+__host__ __device__ inline double expected_near(const GridArgs& a, double r2) {
+    const double gx = ((double)a.dA[0] * (double)a.dB[1] - (double)a.dA[1] * (double)a.dB[0]) * a.nx * a.ny;
+    const double lx = (double)a.lvA[0] * (double)a.lvB[1] - (double)a.lvA[1] * (double)a.lvB[0];
+    double area = (a.npbc_a > 0 && a.npbc_b > 0) ? lx : gx;
+    if (area < 0.0) area = -area;
+    const double n = (double)a.nsites, e = area > 0.0 ? 1.885 * r2 * (double)a.na / area : n;
+    return e < n ? e : n;
+}
+
+// The form of a whole grid: 0 the direct sum, 1 one level of blocks, 2 two levels (LJ only: over the
+// 3.1 A of 32 voxels the tail of a Morse exponential is not resolved by 8 nodes to the relative
+// accuracy of the direct sum).  It depends on the grid, never on the planes a launch stores, and is
+// plain double arithmetic, so host and device agree.
+// Costs are in pair evaluations, of which the card does 2.9e9 per ms (5.8e7: the 20 us any launch
+// takes): direct N per voxel; one level 512 N_far + 4096 N_near per block and 25e3 for its
+// interpolation, but at least one workgroup's own time (8e6 evaluations per ms).  Measured, direct
+// against one level: 20 sites on 160^3 38 / 43 us, 60 on 160^3 96 / 77, 180 on 160x160x48 119 / 47, 540
+// on 83x83x48 at 0.25 A 98 / 152, at 0.2 A and 104x104x60 245 / 115; hence the 0.85.  A second level
+// replaces 7/8 of a block's far evaluations by about 62e3 of interpolation and serial work and has
+// an eighth of the workgroups: measured, one level against two: 300x300x240 voxels with 60 sites 165 /
+// 253 us, 180 sites 253 / 225, 540 655 / 401, 1800 2114 / 722; 160^3 with 1800 538 / 596; 200x200x40
+// with 2304 320 / 357, with 5184 772 / 574.
+__host__ __device__ inline int far_level(const GridArgs& a, int model) {
+    if (a.dC[0] != 0.f || a.dC[1] != 0.f) return 0;
+    const double n = (double)a.nsites, vox = (double)a.nx * a.ny * a.nz;
+    const double near = expected_near(a, near2(a, false));
+    const double per = 512.0 * (n - near) + 4096.0 * near;
+    auto blocks = [&](int b) { return (double)((a.nx + b - 1) / b) * ((a.ny + b - 1) / b) * ((a.nz + b - 1) / b); };
+    double one = blocks(kB) * (per + 25e3);
+    if (one < 362.0 * per) one = 362.0 * per;
+    if (!(one + 5.8e7 < 0.85 * (vox * n + 5.8e7))) return 0;
+    const double nb = blocks(2 * kB), far = (n - expected_near(a, near2(a, true))) * nb;
+    return model == PPM_MODEL_LJ && far >= (nb >= 150.0 ? 1e5 : 4e5) ? 2 : 1;
+}
+
+// A value every lane holds alike, in a scalar register.
+__device__ __forceinline__ float uniform(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+struct Centre {          // centre of a block: FP32 value and the rest of the FP64 one
+    float x, y, z, rx, ry, rz;
+};
+
+__device__ __forceinline__ Centre centre_of(const GridArgs& a, int i0, int j0, int k0, double half) {
+    Centre c;
+    double p[3];
+    for (int q = 0; q < 3; ++q)
+        p[q] = (double)a.p0[q] + (double)a.dA[q] * (i0 + half) + (double)a.dB[q] * (j0 + half) +
+               (double)a.dC[q] * (k0 + half);
+    c.x = uniform((float)p[0]); c.y = uniform((float)p[1]); c.z = uniform((float)p[2]);
+    c.rx = uniform((float)(p[0] - c.x)); c.ry = uniform((float)(p[1] - c.y)); c.rz = uniform((float)(p[2] - c.z));
+    return c;
+}
+
+// Closer than r to the centre c, with every charge of the tip's sites (the tip charge at z offset
+// zo sees the site at S.z - zo; [zlo, zhi] spans 0 and the offsets).  A NaN position is near.
+__device__ __forceinline__ bool is_near(const Site& S, const Centre& c, float r2, float zlo, float zhi) {
+    const float dx = S.x - c.x, dy = S.y - c.y;
+    const float up = S.z - zlo - c.z, lo = S.z - zhi - c.z;      // the interval the charges span
+    const float dz = lo > 0.f ? lo : (up < 0.f ? up : 0.f);
+    return !(dx * dx + dy * dy + dz * dz >= r2);
+}
+
+__device__ __forceinline__ double inv_sqrt(double x) { return 1.0 / sqrt(x); }
+__device__ __forceinline__ float inv_sqrt(float x) { return gc::rsq(x); }
+__device__ __forceinline__ double exp_2(double x) { return exp2(x); }
+__device__ __forceinline__ float exp_2(float x) { return gc::ex2(x); }
+__device__ __forceinline__ float mad(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double mad(double a, double b, double c) { return fma(a, b, c); }
+
+// One site at N points of a column (same dx, dy; dz[k] = oz[k] - sz): f[k] += (Fx, Fy, Fz, E).
+// The pair laws are grid_tile's.  T: type of the terms, ACC: of the sums.
+template <int MODEL, bool HASQ0, int OFF, int N, typename T, typename ACC>
+__device__ __forceinline__ void add_site(const Site& S, const GridArgs& a, T dx, T dy, T sz, const float (&oz)[N],
+                                         ACC (&f)[N][4]) {
+    const T dxy2 = mad(dx, dx, mad(dy, dy, (T)kR2SAFE));
+    const T qq0 = (T)S.q * (T)a.q0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const T dz = (T)oz[k] - sz;
+        const T r2 = mad(dz, dz, dxy2);
+        const T ir = inv_sqrt(r2);
+        const T ir2 = ir * ir;
+        T fr;
+        if (MODEL == PPM_MODEL_LJ) {
+            const T ir6 = ir2 * ir2 * ir2;
+            const T t6 = mad((T)S.c1, ir6, -(T)S.c0), t7 = mad((T)S.c3, ir6, -(T)S.c2);
+            if (HASQ0) {
+                const T ec = qq0 * ir;
+                f[k][3] = mad((ACC)t6, (ACC)ir6, f[k][3] + (ACC)ec);
+                fr = mad(t7, ir6, ec) * ir2;
+            } else {
+                f[k][3] = mad((ACC)t6, (ACC)ir6, f[k][3]);
+                fr = t7 * ir6 * ir2;
+            }
+        } else {
+            const T r = r2 * ir;
+            const T ex = exp_2(mad((T)S.c2, r, (T)S.c0));
+            const T Ae = (T)S.c1 * ex;
+            f[k][3] = mad((ACC)(ex - (T)2), (ACC)Ae, f[k][3]);
+            fr = (T)S.c3 * (Ae * (ex - (T)1)) * ir;
+            if (HASQ0) {
+                const T ec = qq0 * ir;
+                fr = mad(ec, ir2, fr);
+                f[k][3] += (ACC)ec;
+            }
+        }
+        f[k][0] = mad((ACC)fr, (ACC)dx, f[k][0]);
+        f[k][1] = mad((ACC)fr, (ACC)dy, f[k][1]);
+        f[k][2] = mad((ACC)fr, (ACC)dz, f[k][2]);
+    }
+    auto charge = [&](float qf, float zf) {
+        const T qo = (T)S.q * (T)qf, zo = (T)zf;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const T dzo = ((T)oz[k] - sz) + zo;
+            const T iro = inv_sqrt(mad(dzo, dzo, dxy2));
+            const T eo = qo * iro;
+            const T fro = eo * iro * iro;
+            f[k][0] = mad((ACC)fro, (ACC)dx, f[k][0]);
+            f[k][1] = mad((ACC)fro, (ACC)dy, f[k][1]);
+            f[k][2] = mad((ACC)fro, (ACC)dzo, f[k][2]);
+            f[k][3] += (ACC)eo;
+        }
+    };
+    if constexpr (OFF == gc::kOffStatic) {
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            if (o >= a.noff) break;
+            charge(a.qoff[o], a.zoff[o]);
+        }
+    } else if constexpr (OFF == gc::kOffDynamic) {
+        for (int o = 0; o < a.noff; ++o) charge(a.qoff[o], a.zoff[o]);
+    }
+}
+
+// Rank of this thread among the workgroup's threads with flag f (in thread order), and their number;
+// the other flag list g likewise.  Ends with every thread past a barrier; cnt may be reused after
+// the caller's next barrier.
+__device__ __forceinline__ void ranks(bool f, bool g, int (&cnt)[2][4], int& rf, int& nf, int& rg, int& ng) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned long long mf = __ballot(f), mg = __ballot(g), below = (1ull << lane) - 1ull;
+    if (lane == 0) { cnt[0][w] = __popcll(mf); cnt[1][w] = __popcll(mg); }
+    __syncthreads();
+    rf = __popcll(mf & below);
+    rg = __popcll(mg & below);
+    nf = ng = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i < w) { rf += cnt[0][i]; rg += cnt[1][i]; }
+        nf += cnt[0][i];
+        ng += cnt[1][i];
+    }
+}
+
+// Sum over the 4 waves of the node sums f (lane = column y * 8 + x, k = z) into dst[channel][z * 64 + lane].
+template <typename ACC>
+__device__ __forceinline__ void reduce_nodes(Shared& s, const ACC (&f)[kM][4], float (*dst)[kM * kM * kM]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    float* part = &s.b[0][0];                       // 2 x 2048 floats, and the third part in a
+    float* buf[3] = {part, part + 2048, &s.a[0][0]};
+    if (w > 0)
+#pragma unroll
+        for (int k = 0; k < kM; ++k)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) buf[w - 1][(c * kM + k) * 64 + lane] = (float)f[k][c];
+    __syncthreads();
+    float v[kM][4];
+    if (w == 0)
+#pragma unroll
+        for (int k = 0; k < kM; ++k)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int i = (c * kM + k) * 64 + lane;
+                v[k][c] = ((float)f[k][c] + buf[0][i]) + (buf[1][i] + buf[2][i]);
+            }
+    if (dst == nullptr) {                           // into a, which buf[2] is part of: one wave, in order
+        if (w == 0)
+#pragma unroll
+            for (int k = 0; k < kM; ++k)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s.a[c][k * 64 + lane] = v[k][c];
+    } else if (w == 0) {
+#pragma unroll
+        for (int k = 0; k < kM; ++k)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) dst[c][k * 64 + lane] = v[k][c];
+    }
+    __syncthreads();
+}
+
+// a += the polynomial of the 32^3 voxels (top) at the nodes of their block (hx, hy, hz).
+__device__ __forceinline__ void add_top(Shared& s, int hx, int hy, int hz) {
+    const int lane = threadIdx.x & 63, ch = threadIdx.x >> 6;
+    float* t0 = &s.b[0][0] + ch * 512;
+    float* t1 = &s.b[0][0] + 2048 + ch * 512;
+    float v[kM];
+#pragma unroll
+    for (int k = 0; k < kM; ++k) v[k] = s.top[ch][k * 64 + lane];
+#pragma unroll
+    for (int j = 0; j < kM; ++j) {                  // z: lane = (y, x)
+        float o = 0.f;
+#pragma unroll
+        for (int k = 0; k < kM; ++k) o = fmaf(c_tab.sub[hz][j][k], v[k], o);
+        t0[j * 64 + lane] = o;
+    }
+    __syncthreads();
+    const int hi = lane >> 3, lo = lane & 7;
+#pragma unroll
+    for (int k = 0; k < kM; ++k) v[k] = t0[hi * 64 + k * 8 + lo];
+#pragma unroll
+    for (int j = 0; j < kM; ++j) {                  // y: lane = (z, x)
+        float o = 0.f;
+#pragma unroll
+        for (int k = 0; k < kM; ++k) o = fmaf(c_tab.sub[hy][j][k], v[k], o);
+        t1[hi * 64 + j * 8 + lo] = o;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kM; ++k) v[k] = t1[lane * 8 + k];
+#pragma unroll
+    for (int j = 0; j < kM; ++j) {                  // x: lane = (z, y)
+        float o = 0.f;
+#pragma unroll
+        for (int k = 0; k < kM; ++k) o = fmaf(c_tab.sub[hx][j][k], v[k], o);
+        s.a[ch][lane * 8 + j] += o;
+    }
+    __syncthreads();
+}
+
+// f = the polynomial through the node values a at this thread's column (x, y) = (tid & 15, tid >> 4)
+// of the block's voxels: z in registers, then y and x through LDS, 8 planes at a time.
+template <typename ACC>
+__device__ __forceinline__ void interpolate(Shared& s, ACC (&f)[kB][4]) {
+    const int lane = threadIdx.x & 63, ch = threadIdx.x >> 6;
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+    float wx[kM], v[kM], z[kB];
+#pragma unroll
+    for (int k = 0; k < kM; ++k) wx[k] = c_tab.vox[x][k];
+#pragma unroll
+    for (int k = 0; k < kM; ++k) v[k] = s.a[ch][k * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+        z[i] = 0.f;
+#pragma unroll
+        for (int k = 0; k < kM; ++k) z[i] = fmaf(kTab.vox[i][k], v[k], z[i]);
+    }
+    __syncthreads();
+    const int hi = lane >> 3, lo = lane & 7;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s.a[ch][i * 72 + lane] = z[half * 8 + i];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kM; ++k) v[k] = s.a[ch][hi * 72 + k * 8 + lo];
+#pragma unroll
+        for (int j = 0; j < kB; ++j) {              // y: lane = (z, x)
+            float o = 0.f;
+#pragma unroll
+            for (int k = 0; k < kM; ++k) o = fmaf(kTab.vox[j][k], v[k], o);
+            s.b[ch][hi * 136 + j * 8 + lo] = o;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            __builtin_amdgcn_sched_barrier(0);      // keep the reads of later planes out of the registers
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float4* p = reinterpret_cast<const float4*>(&s.b[c][i * 136 + y * 8]);
+                const float4 p0 = p[0], p1 = p[1];
+                float o = wx[0] * p0.x;
+                o = fmaf(wx[1], p0.y, o); o = fmaf(wx[2], p0.z, o); o = fmaf(wx[3], p0.w, o);
+                o = fmaf(wx[4], p1.x, o); o = fmaf(wx[5], p1.y, o); o = fmaf(wx[6], p1.z, o);
+                f[half * 8 + i][c] = (ACC)fmaf(wx[7], p1.w, o);
+            }
+        }
+    }
+}
+
+// Sites [0, nsites) that `keep` accepts, from rank `first` on and at most kList of them, into s.list in
+// site order; returns how many sites `keep` accepts in all.  far(S) is called once per tile of 256
+// sites with the workgroup's other sites in s.tile[0, n).
+template <int MODEL, class KEEP, class FAR>
+__device__ __forceinline__ int collect(Shared& s, const float4* __restrict__ atoms, const float* __restrict__ cpar,
+                                       const GridArgs& a, int first, KEEP keep, FAR far) {
+    int total = 0;
+    for (int t0 = 0; t0 < a.nsites; t0 += 256) {
+        const int i = t0 + (int)threadIdx.x;
+        Site S;
+        bool ok = i < a.nsites, k = false;
+        if (ok) {
+            gc::load_site<MODEL>(atoms, cpar, a, i, S);
+            k = keep(S);
+        }
+        int rk, nk, ro, no;
+        ranks(ok && k, ok && !k, s.cnt, rk, nk, ro, no);
+        const int at = total + rk - first;
+        if (ok && k && at >= 0 && at < kList) s.list[at] = S;
+        if (ok && !k) s.tile[ro] = S;
+        total += nk;
+        __syncthreads();
+        far(no);
+        __syncthreads();
+    }
+    return total;
+}
+
+// The 16^3 blocks of one workgroup of 256 threads: TWO: the 2^3 blocks whose first voxel is (i0, j0, k0),
+// otherwise the one block there.  Voxels with klo <= ic < kend are stored at out[(ic - klo) * ncol + col];
+// base as for grid_tile.  Every thread of the workgroup must call it.
+// ACC: float, or double (pair terms at the nodes and all sums in FP64, terms at the voxels in FP32).
+template <int MODEL, bool HASQ0, int OFF, bool TWO, typename ACC>
+__device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__ atoms, const float* __restrict__ cpar,
+                                           const GridArgs& a, int i0, int j0, int k0, int sub0, int sub1, int klo,
+                                           int kend, float4* __restrict__ out, const float4* base) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float zlo = 0.f, zhi = 0.f;                     // span of the tip charges' z offsets
+#pragma unroll
+    for (int o = 0; o < 4; ++o)
+        if (OFF != gc::kOffNone && o < a.noff) { zlo = fminf(zlo, a.zoff[o]); zhi = fmaxf(zhi, a.zoff[o]); }
+    const float r0 = uniform((float)near2(a, false)), r1 = uniform((float)near2(a, true));      // squared
+
+    // offsets of this lane's column of nodes from a centre, for half-width `half` (voxels)
+    auto node_offsets = [&](const Centre& c, float half, float& ox, float& oy, float (&oz)[kM]) {
+        const int nx = lane & 7, ny = lane >> 3;
+        float ux = 0.f, uy = 0.f;
+#pragma unroll
+        for (int k = 0; k < kM; ++k) {
+            if (k == nx) ux = (float)kNode[k] * half;
+            if (k == ny) uy = (float)kNode[k] * half;
+        }
+        ox = fmaf(a.dA[0], ux, fmaf(a.dB[0], uy, c.rx));
+        oy = fmaf(a.dA[1], ux, fmaf(a.dB[1], uy, c.ry));
+        const float o = fmaf(a.dA[2], ux, fmaf(a.dB[2], uy, c.rz));
+#pragma unroll
+        for (int k = 0; k < kM; ++k) oz[k] = fmaf(a.dC[2], (float)kNode[k] * half, o);
+    };
+
+    bool top = false;
+    int total;
+    if constexpr (TWO) {
+        const Centre c = centre_of(a, i0, j0, k0, kB - 0.5);
+        float ox, oy, oz[kM];
+        node_offsets(c, kB - 0.5f, ox, oy, oz);
+        ACC f[kM][4];
+#pragma unroll
+        for (int k = 0; k < kM; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
+        int nfar = 0;
+        total = collect<MODEL>(s, atoms, cpar, a, 0, [&](const Site& S) { return is_near(S, c, r1, zlo, zhi); },
+                               [&](int n) {
+                                   nfar += n;
+                                   if (wave >= n) return;
+                                   Site Sn = s.tile[wave];      // read one site ahead of use
+                                   for (int j = wave; j < n; j += 4) {
+                                       const Site S = Sn;
+                                       Sn = s.tile[min(j + 4, n - 1)];
+                                       add_site<MODEL, HASQ0, OFF, kM, ACC, ACC>(
+                                           S, a, (ACC)ox - ((ACC)S.x - (ACC)c.x), (ACC)oy - ((ACC)S.y - (ACC)c.y),
+                                           (ACC)S.z - (ACC)c.z, oz, f);
+                                   }
+                               });
+        top = nfar > 0;
+        if (top) reduce_nodes(s, f, s.top);
+    } else {
+        total = collect<MODEL>(s, atoms, cpar, a, 0, [](const Site&) { return true; }, [](int) {});
+    }
+    const int rounds = (total + kList - 1) / kList;
+
+#pragma unroll 1
+    for (int sub = sub0; sub < sub1; ++sub) {
+        const int hx = sub & 1, hy = (sub >> 1) & 1, hz = sub >> 2;
+        const int bi = i0 + hx * kB, bj = j0 + hy * kB, bk = k0 + hz * kB;
+        if (bi >= a.nx || bj >= a.ny || bk >= kend || bk + kB <= klo) continue;
+        const Centre c = centre_of(a, bi, bj, bk, 0.5 * (kB - 1));
+        auto load_round = [&](int r) {              // the sites of this round into the list (one round: there)
+            if (rounds > 1) {
+                const Centre ct = centre_of(a, i0, j0, k0, kB - 0.5);
+                __syncthreads();
+                collect<MODEL>(s, atoms, cpar, a, r * kList,
+                               [&](const Site& S) { return !TWO || is_near(S, ct, r1, zlo, zhi); }, [](int) {});
+            }
+            return min(kList, total - r * kList);
+        };
+        // entries of the list that are near this block (s.near) and not (s.mid); their numbers
+        auto split = [&](int n, int& nmid, int& nnear) {
+            nmid = nnear = 0;
+            for (int i = 0; i < n; i += 256) {
+                const int e = i + (int)threadIdx.x;
+                const bool ok = e < n;
+                const bool nr = ok && is_near(s.list[e], c, r0, zlo, zhi);
+                int rn, nn, rm, nm;
+                __syncthreads();
+                ranks(ok && nr, ok && !nr, s.cnt, rn, nn, rm, nm);
+                if (ok && nr) s.near[nnear + rn] = (unsigned short)e;
+                if (ok && !nr) s.mid[nmid + rm] = (unsigned short)e;
+                nnear += nn;
+                nmid += nm;
+            }
+            __syncthreads();
+        };
+        int nmid = 0, nnear = 0, mids = 0;
+        {
+            float ox, oy, oz[kM];
+            node_offsets(c, 0.5f * (kB - 1), ox, oy, oz);
+            ACC f[kM][4];
+#pragma unroll
+            for (int k = 0; k < kM; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
+            for (int r = 0; r < rounds; ++r) {
+                const int n = load_round(r);
+                split(n, nmid, nnear);
+                if (rounds == 1 && !top && nmid < kMinMid) break;
+                mids += nmid;
+                Site Sn;
+                if (wave < nmid) Sn = s.list[s.mid[wave]];
+                for (int j = wave; j < nmid; j += 4) {
+                    const Site S = Sn;
+                    Sn = s.list[s.mid[min(j + 4, nmid - 1)]];
+                    add_site<MODEL, HASQ0, OFF, kM, ACC, ACC>(S, a, (ACC)ox - ((ACC)S.x - (ACC)c.x),
+                                                             (ACC)oy - ((ACC)S.y - (ACC)c.y),
+                                                             (ACC)S.z - (ACC)c.z, oz, f);
+                }
+            }
+            if (top || mids > 0) reduce_nodes<ACC>(s, f, nullptr);
+        }
+        const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+        ACC f[kB][4];
+        if (top || mids > 0) {
+            if (top) add_top(s, hx, hy, hz);
+            interpolate(s, f);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kB; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
+        }
+        // the voxels' positions as grid_tile has them: a near site's terms are the direct sum's
+        const float fia = (float)(bi + x), fib = (float)(bj + y);
+        const float px = a.p0[0] + a.dA[0] * fia + a.dB[0] * fib + a.dC[0] * (float)bk;
+        const float py = a.p0[1] + a.dA[1] * fia + a.dB[1] * fib + a.dC[1] * (float)bk;
+        float pz[kB];
+#pragma unroll
+        for (int k = 0; k < kB; ++k) pz[k] = a.p0[2] + a.dA[2] * fia + a.dB[2] * fib + a.dC[2] * (float)(bk + k);
+        for (int r = 0; r < rounds; ++r) {
+            if (rounds > 1) {
+                const int n = load_round(r);
+                split(n, nmid, nnear);
+            }
+            auto site = [&](const Site& S) {
+                add_site<MODEL, HASQ0, OFF, kB, float, ACC>(S, a, px - S.x, py - S.y, S.z, pz, f);
+            };
+            auto all = [&](const unsigned short* idx, int n) {
+                if (n == 0) return;
+                Site Sn = s.list[idx[0]];
+                for (int j = 0; j < n; ++j) {
+                    const Site S = Sn;
+                    Sn = s.list[idx[min(j + 1, n - 1)]];
+                    site(S);
+                }
+            };
+            all(s.near, nnear);
+            if (rounds == 1 && mids == 0) all(s.mid, nmid);
+        }
+        if (bi + x < a.nx && bj + y < a.ny) {
+            const int col = (bj + y) * a.nx + bi + x;
+#pragma unroll
+            for (int k = 0; k < kB; ++k) {
+                const int ic = bk + k;
+                if (ic < klo || ic >= kend) continue;
+                float4 v = make_float4((float)f[k][0], (float)f[k][1], (float)f[k][2], (float)f[k][3]);
+                if (base) {
+                    const float4 b = base[(size_t)(ic - klo) * a.ncol + col];
+                    v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
+                }
+                if (a.cap) {
+                    const float renorm = 100.0f / fabsf(v.w);
+                    if (renorm < 1.0f) { v.x *= renorm; v.y *= renorm; v.z *= renorm; v.w *= renorm; }
+                }
+                out[(size_t)(ic - klo) * a.ncol + col] = v;
+            }
+        }
+        __syncthreads();                            // the next block reuses the lists and buffers
+    }
+}
+
+}  // namespace gf
+}  // namespace ppm
