@@ -99,6 +99,7 @@ __device__ rc::TiltArgs tilt_args(const PpmBatchParams& P) {
     t.dtip = P.tip.tipC[3];
     for (int q = 0; q < 4; ++q) { t.k[q] = P.tip.stiffness[q]; t.d0[q] = P.tip.dpos0[q]; }
     t.dt0 = P.tip.relax[0]; t.damp0 = P.tip.relax[1]; t.surf = P.tip.surfFF[0];
+    t.short_ops = rc::spring_in_range(t.k, t.d0);
     return t;
 }
 

@@ -4,11 +4,11 @@
 // Forward (relaxStrokesTiltedMorseDirect, kernels/AFM.cl:1419-1511): the relaxation of
 // relaxStrokesTilted with the trilinear grid sample replaced by the direct, uncapped pair sum
 // over all atoms (getMorse + getCoulombAFM per tip charge site, kernels/AFM.cl:1391-1407),
-// convergence tested before the update.  A scan point is relaxed by a group of G lanes
+// convergence tested before the update.  A scan point's pair sum is split into G running sums
 // (G = 1..64, chosen so that a launch holds about 4 waves per SIMD: a 64x64 scan is only 64
-// waves at one lane per point): each lane sums a strided share of the atoms (held in LDS,
-// <= 128), a butterfly gives every lane of the group the total, and the group runs the FIRE
-// logic in lockstep; groups advance through their z slices independently.  Built with
+// waves at one lane per point) over strided shares of the atoms (held in LDS, <= 128), one or two
+// of them to a lane; a butterfly gives every lane of the group the total, and the group runs the
+// FIRE logic in lockstep; groups advance through their z slices independently.  Built with
 // -ffp-contract=off: the FP32 operations follow the reference formulas as written (with G = 1
 // the atoms are also summed in the reference's order).
 //
@@ -34,6 +34,7 @@ constexpr int kAdjBlock = 256;
 struct DirectArgs {
     int na, nsite;
     float Qs[4], QZs[4];     // non-zero tip charge sites only, Qs scaled by COULOMB_CONST
+    int tame;                // every |QZs| below kTame
 };
 
 __device__ __forceinline__ void load_atoms(const float4* __restrict__ atoms, const float4* __restrict__ cms, int na,
@@ -45,65 +46,105 @@ __device__ __forceinline__ void load_atoms(const float4* __restrict__ atoms, con
     __syncthreads();
 }
 
-// Pair sum of one lane of a G-lane group: atoms sub, sub+G, sub+2G, ... then a butterfly over
-// the group, after which every lane of the group holds the same total (FP32 addition is
-// commutative, so both partners of each exchange compute the identical sum).
-template <int G>
+// Coordinates below this (A) leave every r^2 + R2SAFE in [1e-4, 2^60], the range of ppm_rn.hpp.
+constexpr float kTame = 1e8f;
+
+// Pair sum of a point, shared by a group of P lanes: G running sums (sum s: atoms s, s + G, s + 2G, ...),
+// G / P of them in each lane, then the butterfly over the G sums (distances G/2, ..., 1), the first steps
+// of it within the lane, after which every lane of the group holds the same total.  The order of the
+// additions is that of G lanes with one sum each, so the bits do not depend on P (FP32 addition is
+// commutative).  Atoms past na are null (k_direct_relax): they add zeros.
+// RN: the coordinates are tame, so roots and reciprocals take their short forms (same bits): 80 instead
+// of 116 VALU instructions per atom with one charge site.
+template <int G, int P, bool RN>
 __device__ __forceinline__ float4 direct_fe_group(const float4* __restrict__ A, const float4* __restrict__ M,
                                                   const DirectArgs& d, int sub, float x, float y, float z) {
-    float4 fe = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int j = sub; j < d.na; j += G) {
-        const float4 a = A[j];
-        const float4 m = M[j];
-        const float dx = x - a.x, dy = y - a.y, dz = z - a.z;
-        const float r = sqrtf(dx * dx + dy * dy + dz * dz + kR2SAFE);
-        const float ex = expf(m.z * (r - m.x));
-        const float E = m.y * ex * (ex - 2.0f);
-        const float fr = -m.y * ex * (ex - 1.0f) * 2.0f * m.z;
-        const float fq = fr / r;
-        fe.x += dx * fq; fe.y += dy * fq; fe.z += dz * fq; fe.w += E;
-        for (int k = 0; k < d.nsite; ++k) {
-            const float kx = x - a.x, ky = y - a.y, kz = (z + d.QZs[k]) - a.z;
-            const float ir2 = 1.0f / (kx * kx + ky * ky + kz * kz + kR2SAFE);
-            const float Ec = a.w * sqrtf(ir2);
-            const float e2 = Ec * ir2;
-            fe.x += (kx * e2) * d.Qs[k]; fe.y += (ky * e2) * d.Qs[k]; fe.z += (kz * e2) * d.Qs[k];
-            fe.w += Ec * d.Qs[k];
+    constexpr int R = G / P;
+    float4 fe[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) fe[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = sub; j - sub < d.na; j += G) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (!RN && j + r * P >= d.na) continue;    // a null atom's terms are 0 at a finite distance only
+            const float4 a = A[j + r * P];
+            const float4 m = M[j + r * P];
+            const float dx = x - a.x, dy = y - a.y, dz = z - a.z;
+            const float r2 = dx * dx + dy * dy + dz * dz + kR2SAFE;
+            const float rr = RN ? sqrt_rn(r2) : sqrtf(r2);
+            const float ex = expf(m.z * (rr - m.x));
+            const float E = m.y * ex * (ex - 2.0f);
+            const float fr = -m.y * ex * (ex - 1.0f) * 2.0f * m.z;
+            const float fq = fr / rr;
+            fe[r].x += dx * fq; fe[r].y += dy * fq; fe[r].z += dz * fq; fe[r].w += E;
+            for (int k = 0; k < d.nsite; ++k) {
+                float kz = dz, k2 = r2;                 // a charge at z offset 0 shares the distance
+                if (d.QZs[k] != 0.f) {
+                    kz = (z + d.QZs[k]) - a.z;
+                    k2 = dx * dx + dy * dy + kz * kz + kR2SAFE;
+                }
+                const float ir2 = RN ? rcp_rn(k2) : 1.0f / k2;
+                const float Ec = a.w * (RN ? sqrt_rn(ir2) : sqrtf(ir2));
+                const float e2 = Ec * ir2;
+                fe[r].x += (dx * e2) * d.Qs[k]; fe[r].y += (dy * e2) * d.Qs[k]; fe[r].z += (kz * e2) * d.Qs[k];
+                fe[r].w += Ec * d.Qs[k];
+            }
         }
     }
 #pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) {
-        fe.x += __shfl_xor(fe.x, off, G);
-        fe.y += __shfl_xor(fe.y, off, G);
-        fe.z += __shfl_xor(fe.z, off, G);
-        fe.w += __shfl_xor(fe.w, off, G);
-    }
-    return fe;
+    for (int h = R / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int r = 0; r < h; ++r) {
+            fe[r].x += fe[r + h].x; fe[r].y += fe[r + h].y; fe[r].z += fe[r + h].z; fe[r].w += fe[r + h].w;
+        }
+    return make_float4(group_sum<P>(fe[0].x), group_sum<P>(fe[0].y), group_sum<P>(fe[0].z), group_sum<P>(fe[0].w));
 }
 
-// G lanes per scan point (G = 1: one lane per point, the atoms summed in order).  The group's
-// lanes share every branch (same data), so the shuffles only read active lanes.
-template <int G>
+template <int G, int P>
+struct DirectSample {
+    const float4 *A, *M;
+    const DirectArgs& d;
+    int sub;
+    bool tame;
+    __device__ __forceinline__ float4 operator()(float x, float y, float z) const {
+        return tame && fabsf(x) + fabsf(y) + fabsf(z) < kTame ? direct_fe_group<G, P, true>(A, M, d, sub, x, y, z)
+                                                              : direct_fe_group<G, P, false>(A, M, d, sub, x, y, z);
+    }
+    __device__ __forceinline__ void begin() const {}
+    __device__ __forceinline__ void end() const {}
+};
+
+// P lanes per scan point (P = 1: one lane per point), G running sums.  The group's lanes share every
+// branch (same data), so the exchanges only read active lanes.
+template <int G, int P>
 __global__ __launch_bounds__(256) void k_direct_relax(const float4* __restrict__ atoms, const float4* __restrict__ cms,
                                                       DirectArgs d, const float4* __restrict__ pts, rc::TiltArgs p,
                                                       float4* __restrict__ FEs, float4* __restrict__ PPs) {
     __shared__ float4 A[kMaxAtoms], M[kMaxAtoms];
-    load_atoms(atoms, cms, d.na, A, M);        // every lane takes part before any leaves
+    bool tame = d.tame != 0;
+    for (int i = threadIdx.x; i < kMaxAtoms; i += blockDim.x) {      // null atoms past na
+        const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 a = i < d.na ? atoms[i] : none;
+        tame = tame && fabsf(a.x) < kTame && fabsf(a.y) < kTame && fabsf(a.z) < kTame;
+        A[i] = a;
+        M[i] = i < d.na ? cms[i] : none;
+    }
+    tame = __syncthreads_and(tame);
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ip = t / G, sub = t - ip * G;
+    const int ip = t / P, sub = t - ip * P;
     if (ip >= p.n_scan) return;                // whole groups leave together
-    const float4 P = pts[ip];
-    auto smp = [&](float x, float y, float z) { return direct_fe_group<G>(A, M, d, sub, x, y, z); };
+    const float4 Q = pts[ip];
+    DirectSample<G, P> smp{A, M, d, sub, tame != 0};
     const size_t o = (size_t)ip * p.nz;
-    rc::relax_tilted_lane_src<G>(smp, mk3(P.x, P.y, P.z), p, FEs + o, PPs ? PPs + o : nullptr, sub);
+    rc::relax_tilted_lane_src<P>(smp, mk3(Q.x, Q.y, Q.z), p, FEs + o, PPs ? PPs + o : nullptr, sub);
 }
 
-// Lanes per scan point: enough groups for about 4 waves per SIMD (1024 SIMDs), at most one
-// lane per atom, a power of two in [1, 64].
+// Running sums per scan point: at one lane for each, enough groups for about 4 waves per SIMD (1024
+// SIMDs), at most one per atom, a power of two in [1, 64].
+constexpr long long kDirectLanes = 4LL * 1024 * 64;
 int direct_group(int n_scan, int na) {
-    const long long want = 4LL * 1024 * 64;
     int g = 1;
-    while (g < 64 && (long long)n_scan * g * 2 <= want && g < na) g *= 2;
+    while (g < 64 && (long long)n_scan * g * 2 <= kDirectLanes && g < na) g *= 2;
     return g;
 }
 
@@ -376,10 +417,12 @@ int launch_direct_relax(const float* atoms, const float* cms, int na, const floa
                         float* PPs, hipStream_t stream) {
     DirectArgs d{};
     d.na = na;
+    d.tame = 1;
     for (int k = 0; k < 4; ++k)
         if (Qs[k] != 0.f) {
             d.Qs[d.nsite] = Qs[k] * kCOULOMB;
             d.QZs[d.nsite] = QZs[k];
+            d.tame = d.tame && fabsf(QZs[k]) < kTame;
             ++d.nsite;
         }
     rc::TiltArgs p{};
@@ -389,22 +432,31 @@ int launch_direct_relax(const float* atoms, const float* cms, int na, const floa
     p.dtip = tip.tipC[3];
     for (int q = 0; q < 4; ++q) { p.k[q] = tip.stiffness[q]; p.d0[q] = tip.dpos0[q]; }
     p.dt0 = tip.relax[0]; p.damp0 = tip.relax[1]; p.surf = tip.surfFF[0];
+    p.short_ops = rc::spring_in_range(p.k, p.d0);
     const int g = direct_group(n_scan, na);
-    const dim3 blocks((unsigned)(((long long)n_scan * g + 255) / 256));
     const float4* A = reinterpret_cast<const float4*>(atoms);
     const float4* M = reinterpret_cast<const float4*>(cms);
     const float4* S = reinterpret_cast<const float4*>(pts);
     float4* F = reinterpret_cast<float4*>(FEs);
     float4* Q = reinterpret_cast<float4*>(PPs);
+    // Two sums in each lane from 3.5 waves per SIMD on, at G = 32 and 64: with half the waves each has two
+    // independent chains, and the FIRE logic runs in half the lanes.  Forward of 100 atoms and 60 heights, ms
+    // with 1 | 2 sums in a lane: 64 x 64 points (G = 64) 0.714 | 0.669, 85 x 85 (G = 32) 0.974 | 0.962; below,
+    // the card wants the waves: 40 x 40 points 0.468 | 0.588; and with G <= 16 one sum a lane was never slower.
+    const bool two = g >= 32 && (long long)n_scan * g * 8 >= 7 * kDirectLanes;
+#define PPM_DIRECT(G, P)                                                                                            \
+    hipLaunchKernelGGL((k_direct_relax<G, P>), dim3((unsigned)(((long long)n_scan * (P) + 255) / 256)), dim3(256), 0, \
+                       stream, A, M, d, S, p, F, Q)
     switch (g) {
-        case 1: hipLaunchKernelGGL(k_direct_relax<1>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        case 2: hipLaunchKernelGGL(k_direct_relax<2>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        case 4: hipLaunchKernelGGL(k_direct_relax<4>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        case 8: hipLaunchKernelGGL(k_direct_relax<8>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        case 16: hipLaunchKernelGGL(k_direct_relax<16>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        case 32: hipLaunchKernelGGL(k_direct_relax<32>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
-        default: hipLaunchKernelGGL(k_direct_relax<64>, blocks, dim3(256), 0, stream, A, M, d, S, p, F, Q); break;
+        case 1: PPM_DIRECT(1, 1); break;
+        case 2: PPM_DIRECT(2, 2); break;
+        case 4: PPM_DIRECT(4, 4); break;
+        case 8: PPM_DIRECT(8, 8); break;
+        case 16: PPM_DIRECT(16, 16); break;
+        case 32: if (two) PPM_DIRECT(32, 16); else PPM_DIRECT(32, 32); break;
+        default: if (two) PPM_DIRECT(64, 32); else PPM_DIRECT(64, 64); break;
     }
+#undef PPM_DIRECT
     return check_launch("direct_relax");
 }
 

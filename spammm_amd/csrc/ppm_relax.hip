@@ -43,7 +43,9 @@ constexpr size_t kStageBytes = 8 * 64 * sizeof(float4);
 // FAST: identity tip frame and grid axes along the world axes (the form of every untilted scan),
 // which skips the rotations and the off-axis texture-coordinate terms (same results).
 // LDSST (G = 1): the FEs and PPs runs are staged in LDS (kStageBytes per workgroup) instead of
-// registers: 12.7 % fewer VALU instructions on the flake scan, 91 instead of 114 VGPRs.
+// registers: 12.7 % fewer VALU instructions on the flake scan, 96 instead of 123 VGPRs.
+// Bound by its waves' instruction chains (grid reads hit L2): 256 x 256 points, 60 heights and at most 100
+// steps take 2.27 ms (2.39 with IEEE roots and quotients and LDS exchanges between the lanes of a group).
 template <int G, bool FAST, bool LDSST = false>
 __global__ __launch_bounds__(64) void k_relax_tilted(GridDev g, const float4* __restrict__ pts, TiltArgs p,
                                                      float4* __restrict__ FEs, float4* __restrict__ PPs,
@@ -66,11 +68,9 @@ __global__ __launch_bounds__(64) void k_relax_tilted(GridDev g, const float4* __
         relax_tilted_lane<true, FAST, LDSST>(g, mk3(P.x, P.y, P.z), p, FEs + o, PPs ? PPs + o : nullptr, dp, row,
                                              col, stage);
     } else {
-        GroupCell<G> cell;
-        cell.reset();
-        auto smp = [&](float x, float y, float z) { return sample_group<G, FAST>(g, cell, sub, x, y, z); };
-        relax_tilted_lane_src<G, decltype(smp), true, FAST>(smp, mk3(P.x, P.y, P.z), p, FEs + o,
-                                                            PPs ? PPs + o : nullptr, sub, dp, row, col);
+        GridSample<G, FAST> smp{g, sub};
+        relax_tilted_lane_src<G, GridSample<G, FAST>, true, FAST>(smp, mk3(P.x, P.y, P.z), p, FEs + o,
+                                                                  PPs ? PPs + o : nullptr, sub, dp, row, col);
     }
 }
 
@@ -104,15 +104,17 @@ struct StrokeArgs {
     float dTip[3];
     float k[4], d0[4];
     float dt0, damp0;
+    int short_ops;          // as in TiltArgs
 };
 
 // relaxStrokes with optional displacement and PP outputs, for one scan point; `smp(x,y,z)` is the
 // trilinear sample (one lane's cell cache, or a lane group's channel-split sample), `writer` the
 // lane that stores (all lanes of a group hold the same state).
-template <class SAMPLE>
-__device__ __forceinline__ void strokes_lane(SAMPLE& smp, int ip, const float4* __restrict__ pts,
-                                             const StrokeArgs& p, float4* __restrict__ FEs,
-                                             float4* __restrict__ disps, float4* __restrict__ PPs, bool writer) {
+// RN: as relax_tilted_column.
+template <bool RN, class SAMPLE>
+__device__ __forceinline__ bool strokes_column(SAMPLE& smp, int ip, const float4* __restrict__ pts,
+                                               const StrokeArgs& p, float4* __restrict__ FEs,
+                                               float4* __restrict__ disps, float4* __restrict__ PPs, bool writer) {
     const f3 dTip = ld3(p.dTip);
     const float4 P = pts[ip];
     f3 tip = mk3(P.x, P.y, P.z);
@@ -121,13 +123,14 @@ __device__ __forceinline__ void strokes_lane(SAMPLE& smp, int ip, const float4* 
     const float dtmax = dt, dtmin = dtmax * 0.1f, damp0 = damp;
     f3 v = mk3(0.f, 0.f, 0.f);
     int it = 0, iz = 0;
+    MidRange<RN> mr;
     size_t o = (size_t)ip * p.nz;
     while (true) {
         const float4 fe = smp(pos.x, pos.y, pos.z);
-        const f3 ft = tipForce(mk3(pos.x - tip.x, pos.y - tip.y, pos.z - tip.z), p.k, p.d0);
+        const f3 ft = tipForce<RN>(mk3(pos.x - tip.x, pos.y - tip.y, pos.z - tip.z), p.k, p.d0, mr);
         const f3 f = mk3(fe.x + ft.x, fe.y + ft.y, fe.z + ft.z);
         const float ff = dot3(f, f);
-        v = integrate(p.damped, f, v, dt, damp, dtmin, dtmax, damp0);
+        v = integrate<RN>(p.damped, f, v, dt, damp, dtmin, dtmax, damp0, mr);
         v = mk3(v.x + f.x * dt, v.y + f.y * dt, v.z + f.z * dt);
         pos = mk3(pos.x + v.x * dt, pos.y + v.y * dt, pos.z + v.z * dt);
         const bool conv = ff < p.f2conv;
@@ -148,9 +151,19 @@ __device__ __forceinline__ void strokes_lane(SAMPLE& smp, int ip, const float4* 
             pos = mk3(pos.x + dTip.x, pos.y + dTip.y, pos.z + dTip.z);
             v = mk3(0.f, 0.f, 0.f);
             it = 0;
-            if (++iz >= p.nz) break;
+            if (++iz >= p.nz || mr.out()) break;
         }
     }
+    return !mr.out();
+}
+template <class SAMPLE>
+__device__ __forceinline__ void strokes_lane(SAMPLE& smp, int ip, const float4* __restrict__ pts,
+                                             const StrokeArgs& p, float4* __restrict__ FEs,
+                                             float4* __restrict__ disps, float4* __restrict__ PPs, bool writer) {
+    smp.begin();
+    if (p.short_ops && strokes_column<true>(smp, ip, pts, p, FEs, disps, PPs, writer)) return;
+    smp.begin();
+    strokes_column<false>(smp, ip, pts, p, FEs, disps, PPs, writer);
 }
 
 // relaxStrokes; G lanes per scan point as k_relax_tilted (results identical to G = 1).
@@ -161,17 +174,8 @@ __global__ __launch_bounds__(64) void k_relax_strokes(GridDev g, const float4* _
     int sub;
     const int ip = group_point<G>(p.n_scan, p.scan_ny, sub);
     if (ip < 0) return;                       // whole groups leave together
-    if constexpr (G == 1) {
-        Cell cell;
-        cell.reset();
-        auto smp = [&](float x, float y, float z) { return sample(g, cell, x, y, z); };
-        strokes_lane(smp, ip, pts, p, FEs, disps, PPs, true);
-    } else {
-        GroupCell<G> cell;
-        cell.reset();
-        auto smp = [&](float x, float y, float z) { return sample_group<G>(g, cell, sub, x, y, z); };
-        strokes_lane(smp, ip, pts, p, FEs, disps, PPs, sub == 0);
-    }
+    GridSample<G, false> smp{g, sub};
+    strokes_lane(smp, ip, pts, p, FEs, disps, PPs, sub == 0);
 }
 
 struct Strokes2DArgs {
@@ -653,6 +657,7 @@ int launch_relax_tilted(const float* grid, const PpmGridSpec& s, const float* pt
     p.dtip = tip.tipC[3];
     for (int q = 0; q < 4; ++q) { p.k[q] = tip.stiffness[q]; p.d0[q] = tip.dpos0[q]; }
     p.dt0 = tip.relax[0]; p.damp0 = tip.relax[1]; p.surf = tip.surfFF[0];
+    p.short_ops = spring_in_range(p.k, p.d0);
     const int G = ctl.lanes > 0 ? ctl.lanes : relax_group(n_scan);
     const dim3 blocks((unsigned)group_waves(n_scan, ctl.scan_ny, G));
     GridDev gd = make_grid(grid, s);
@@ -695,6 +700,7 @@ int launch_relax_strokes(const float* grid, const PpmGridSpec& s, const float* p
     for (int q = 0; q < 3; ++q) p.dTip[q] = dTip[q];
     for (int q = 0; q < 4; ++q) { p.k[q] = stiffness[q]; p.d0[q] = dpos0[q]; }
     p.dt0 = relax[0]; p.damp0 = relax[1];
+    p.short_ops = spring_in_range(p.k, p.d0);
     const int G = ctl.lanes > 0 ? ctl.lanes : relax_group(n_scan);
     const dim3 blocks((unsigned)group_waves(n_scan, ctl.scan_ny, G));
     const GridDev gd = make_grid(grid, s);

@@ -7,6 +7,8 @@
 #include <type_traits>
 
 #include "ppm_common.hpp"
+#include "ppm_lanes.hpp"
+#include "ppm_rn.hpp"
 
 namespace ppm {
 namespace rc {
@@ -29,8 +31,9 @@ struct GridDev {
 // are a function of them (axis_index), so they are only computed when one changes.
 struct Cell {
     float fi, fj, fk;  // floors of the cached cell; -2 = empty
+    bool out;          // a sampled cell lay outside the stored planes
     float4 c[8];       // corners 000,100,010,110,001,101,011,111
-    __device__ void reset() { fi = fj = fk = -2.0f; }
+    __device__ void reset() { fi = fj = fk = -2.0f; out = false; }
 };
 
 // REPEAT addressing of one axis: the interpolation weight a and the floor fl of the texel
@@ -59,9 +62,9 @@ __host__ __device__ inline bool small_grid(const GridDev& g) {
 
 // Element offsets of the 4 corner rows (k0,j0), (k0,j1), (k1,j0), (k1,j1) of the cell with floors
 // (fa, fb, fc) in the stored planes, and its two x indices.  A cell outside the stored planes sets
-// *g.flag (from lane `flag_lane`) and is clamped into them.  O32: 32-bit offsets (small_grid).
+// `out` and is clamped into them.  O32: 32-bit offsets (small_grid).
 template <bool O32>
-__device__ __forceinline__ void cell_rows(const GridDev& g, float fa, float fb, float fc, bool flag_lane, int& i0,
+__device__ __forceinline__ void cell_rows(const GridDev& g, float fa, float fb, float fc, bool& out, int& i0,
                                           int& i1, typename std::conditional<O32, unsigned, size_t>::type (&r)[4]) {
     using T = typename std::conditional<O32, unsigned, size_t>::type;
     int j0, j1, k0, k1;
@@ -71,7 +74,7 @@ __device__ __forceinline__ void cell_rows(const GridDev& g, float fa, float fb, 
     k0 -= g.klo;
     k1 -= g.klo;
     if ((unsigned)k0 >= (unsigned)g.nzw || (unsigned)k1 >= (unsigned)g.nzw) {
-        if (g.flag && flag_lane) atomicOr(g.flag, 1);
+        out = true;
         k0 = min(max(k0, 0), g.nzw - 1);
         k1 = min(max(k1, 0), g.nzw - 1);
     }
@@ -123,7 +126,7 @@ __device__ __forceinline__ float4 sample(const GridDev& g, Cell& C, float px, fl
         C.fi = fa; C.fj = fb; C.fk = fc;
         int i0, i1;
         typename std::conditional<FAST, unsigned, size_t>::type r[4];
-        cell_rows<FAST>(g, fa, fb, fc, true, i0, i1, r);
+        cell_rows<FAST>(g, fa, fb, fc, C.out, i0, i1, r);
         if constexpr (FAST) {
             const char* base = reinterpret_cast<const char*>(g.data);
 #pragma unroll
@@ -145,8 +148,9 @@ __device__ __forceinline__ float4 sample(const GridDev& g, Cell& C, float px, fl
 template <int G>
 struct GroupCell {
     float fi, fj, fk;
+    bool out;
     float c[4 / G][8];
-    __device__ void reset() { fi = fj = fk = -2.0f; }
+    __device__ void reset() { fi = fj = fk = -2.0f; out = false; }
 };
 
 template <int G, bool FAST = false>
@@ -161,7 +165,7 @@ __device__ __forceinline__ float4 sample_group(const GridDev& g, GroupCell<G>& C
         C.fi = fa; C.fj = fb; C.fk = fc;
         int i0, i1;
         typename std::conditional<FAST, unsigned, size_t>::type r[4];
-        cell_rows<FAST>(g, fa, fb, fc, sub == 0, i0, i1, r);
+        cell_rows<FAST>(g, fa, fb, fc, C.out, i0, i1, r);
         if constexpr (FAST) {
             const char* base = reinterpret_cast<const char*>(g.data);
             const unsigned ch = (unsigned)(sub * NC * 4);       // this lane's channels within a texel
@@ -196,11 +200,36 @@ __device__ __forceinline__ float4 sample_group(const GridDev& g, GroupCell<G>& C
         const float hi = (f[4] * ma + f[5] * a) * mb + (f[6] * ma + f[7] * a) * b;
         v[q] = lo * mc + hi * c;
     }
-    float o[4];
-#pragma unroll
-    for (int ch = 0; ch < 4; ++ch) o[ch] = __shfl(v[ch % NC], ch / NC, G);
-    return make_float4(o[0], o[1], o[2], o[3]);
+    return make_float4(from_lane<G, 0>(v[0]), from_lane<G, 1 / NC>(v[1 % NC]), from_lane<G, 2 / NC>(v[2 % NC]),
+                       from_lane<G, 3 / NC>(v[3 % NC]));
 }
+
+// The sample of a relaxation.  begin() before each try of a column, end() once it is finished: a window's
+// flag is raised by the finished try alone.
+template <int G, bool FAST>
+struct GridSample {
+    const GridDev& g;
+    int sub;
+    GroupCell<G> cell;
+    __device__ __forceinline__ float4 operator()(float x, float y, float z) {
+        return sample_group<G, FAST>(g, cell, sub, x, y, z);
+    }
+    __device__ __forceinline__ void begin() { cell.reset(); }
+    __device__ __forceinline__ void end() const {
+        if (cell.out && g.flag && sub == 0) atomicOr(g.flag, 1);
+    }
+};
+template <bool FAST>
+struct GridSample<1, FAST> {
+    const GridDev& g;
+    int sub;
+    Cell cell;
+    __device__ __forceinline__ float4 operator()(float x, float y, float z) { return sample<FAST>(g, cell, x, y, z); }
+    __device__ __forceinline__ void begin() { cell.reset(); }
+    __device__ __forceinline__ void end() const {
+        if (cell.out && g.flag) atomicOr(g.flag, 1);
+    }
+};
 
 __device__ __forceinline__ float dot3(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ __forceinline__ f3 rotMat(f3 v, f3 a, f3 b, f3 c) { return mk3(dot3(v, a), dot3(v, b), dot3(v, c)); }
@@ -208,36 +237,84 @@ __device__ __forceinline__ f3 rotMatT(f3 v, f3 a, f3 b, f3 c) {
     return mk3(a.x * v.x + b.x * v.y + c.x * v.z, a.y * v.x + b.y * v.y + c.y * v.z,
                a.z * v.x + b.z * v.y + c.z * v.z);
 }
-__device__ __forceinline__ f3 tipForce(f3 d, const float* k, const float* d0) {
-    float r = sqrtf(dot3(d, d));
-    r = fmaxf(r, 1e-10f);
-    const float s = (k[3] * (r - d0[3])) / r;
+// The operands of a relaxation's roots and quotients so far.  RN: they take the forms of ppm_rn.hpp, which
+// hold in the middle of the exponent range: r^2 in [2^-94, 2^60], v.v = 0 or in it, f.f + kF2SAFE <= 2^60,
+// the quotient of the two 0 or >= 2^-94.  out() tells whether one lay outside (a NaN does); the caller then
+// relaxes the column again with RN = false, the IEEE forms, which have the same bits inside.  Two integer
+// minima and maxima of the bits a step and no branch: with a test and a branch in every step the short forms
+// saved nothing (relaxStrokes of 100 x 80 points and 31 heights: 0.62 ms with the IEEE forms, 0.62 with the
+// branch, 0.55 as this).
+template <bool RN>
+struct MidRange {
+    static constexpr unsigned kLo = 0x10800000u, kHi = 0x5d800000u;      // bits of 2^-94 and 2^60
+    unsigned lo = ~0u, hi = 0u;
+    __device__ __forceinline__ void root(float rr) {
+        if (RN) {
+            lo = min(lo, __float_as_uint(rr));
+            hi = max(hi, __float_as_uint(rr));
+        }
+    }
+    __device__ __forceinline__ void ratio(float vv, float fs, float q) {    // 0 wraps to the top
+        if (RN) {
+            lo = min(lo, min(__float_as_uint(vv) - 1u, __float_as_uint(q) - 1u));
+            hi = max(hi, max(__float_as_uint(vv), __float_as_uint(fs)));
+        }
+    }
+    __device__ __forceinline__ bool out() const { return RN && (lo < kLo || hi > kHi); }
+};
+// Where MidRange's ranges cover the spring as well: its constant 0 or in 2^+-30, its length in it or 0 with
+// the tip's rest position away from the anchor, so that k (r - l) is 0 or at least 2^-94.
+__host__ __device__ inline bool spring_in_range(const float* k, const float* d0) {
+    auto mid = [](float v) { return fabsf(v) >= 0x1p-30f && fabsf(v) <= 0x1p30f; };
+    return (k[3] == 0.f || mid(k[3])) && (d0[3] == 0.f || mid(d0[3])) && (mid(d0[0]) || mid(d0[1]) || mid(d0[2]));
+}
+template <bool RN>
+__device__ __forceinline__ f3 tipForce(f3 d, const float* k, const float* d0, MidRange<RN>& mr) {
+    const float rr = dot3(d, d);
+    float r, s;
+    if (RN) {
+        r = sqrt_rn(rr);
+        s = div_rn(k[3] * (r - d0[3]), r);
+        mr.root(rr);
+    } else {
+        r = fmaxf(sqrtf(rr), 1e-10f);
+        s = (k[3] * (r - d0[3])) / r;
+    }
     return mk3((d.x - d0[0]) * k[0] + d.x * s, (d.y - d0[1]) * k[1] + d.y * s, (d.z - d0[2]) * k[2] + d.z * s);
 }
-// update_FIRE: returns the new velocity, updates dt and damp.
-__device__ __forceinline__ f3 fire(f3 f, f3 v, float& dt, float& damp, float dtmin, float dtmax, float damp0) {
+// update_FIRE: returns the new velocity, updates dt and damp.  Its two outcomes are selected, not branched
+// to: some lane of a wave takes each on nearly every step.
+template <bool RN>
+__device__ __forceinline__ f3 fire(f3 f, f3 v, float& dt, float& damp, float dtmin, float dtmax, float damp0,
+                                   MidRange<RN>& mr) {
     const float ff = dot3(f, f), vv = dot3(v, v), vf = dot3(v, f);
-    if (vf < 0.0f) {
-        dt = fmaxf(dtmin, dt * kFTDEC);
-        damp = damp0;
-        return mk3(0.f, 0.f, 0.f);
+    const bool back = vf < 0.0f;
+    const float cv = 1.0f - damp, fs = ff + kF2SAFE;
+    float cf;
+    if (RN) {
+        const float q = div_rn(vv, fs);
+        cf = damp * sqrt_rn<true>(q);
+        mr.ratio(vv, fs, q);
+    } else {
+        cf = damp * sqrtf(vv / fs);
     }
-    const float cv = 1.0f - damp;
-    const float cf = damp * sqrtf(vv / (ff + kF2SAFE));
-    dt = fminf(dtmax, dt * kFTINC);
-    damp = damp * kFDAMP;
-    return mk3(v.x * cv + f.x * cf, v.y * cv + f.y * cf, v.z * cv + f.z * cf);
+    const float dtd = fmaxf(dtmin, dt * kFTDEC), dtu = fminf(dtmax, dt * kFTINC);
+    dt = back ? dtd : dtu;
+    damp = back ? damp0 : damp * kFDAMP;
+    const f3 u = mk3(v.x * cv + f.x * cf, v.y * cv + f.y * cf, v.z * cv + f.z * cf);
+    return mk3(back ? 0.f : u.x, back ? 0.f : u.y, back ? 0.f : u.z);
 }
 // The integrator step before `v += f dt; pos += v dt`: update_FIRE, or the damped-velocity
 // update `v *= (1 - damp)` of the reference's OPT_FIRE=0 build (kernels/AFM.cl:378-382), whose dt
 // and damp stay at their initial values.
+template <bool RN>
 __device__ __forceinline__ f3 integrate(bool damped, f3 f, f3 v, float& dt, float& damp, float dtmin, float dtmax,
-                                        float damp0) {
+                                        float damp0, MidRange<RN>& mr) {
     if (damped) {
         const float cv = 1.0f - damp;
         return mk3(v.x * cv, v.y * cv, v.z * cv);
     }
-    return fire(f, v, dt, damp, dtmin, dtmax, damp0);
+    return fire<RN>(f, v, dt, damp, dtmin, dtmax, damp0, mr);
 }
 
 __device__ __forceinline__ bool finite4(float4 v) {
@@ -286,6 +363,7 @@ struct TiltArgs {
     float A[3], B[3], C[3], dtip;
     float k[4], d0[4];
     float dt0, damp0, surf;
+    int short_ops;          // spring_in_range(k, d0): columns are tried with MidRange's short forms
 };
 
 // Output staging of one lane: the newest (up to 4) states of its column are held in registers
@@ -339,13 +417,12 @@ struct DfOut {
 // and the z-only shifts (tip step, surface force) leave x and y alone, for finite values up to
 // the sign of a zero, so they are skipped: the same results with ~30 fewer instructions per
 // FIRE step.
-template <int G, class SAMPLE, bool STAGE = true, bool IDF = false, bool LDSST = false>
-__device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, const TiltArgs& p,
-                                                      float4* __restrict__ FEs, float4* __restrict__ PPs,
-                                                      int sub = 0, const DfOut* dfo = nullptr,
-                                                      float* __restrict__ dfrow = nullptr,
-                                                      float* __restrict__ fz_lds = nullptr,
-                                                      float4* __restrict__ stage = nullptr) {
+// RN: the short roots and quotients (MidRange); false is returned, with the outputs unfinished, if an
+// operand was out of their range.
+template <bool RN, int G, class SAMPLE, bool STAGE, bool IDF, bool LDSST>
+__device__ __forceinline__ bool relax_tilted_column(SAMPLE& sample, f3 start, const TiltArgs& p,
+                                                    float4* __restrict__ FEs, float4* __restrict__ PPs, int sub,
+                                                    float* __restrict__ fz_lds, float4* __restrict__ stage) {
     static_assert(!LDSST || (STAGE && G == 1), "LDS staging is built for one lane per point");
     const f3 A = ld3(p.A), B = ld3(p.B), C = ld3(p.C);
     const f3 dTip = mk3(C.x * p.dtip, C.y * p.dtip, C.z * p.dtip);
@@ -365,19 +442,20 @@ __device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, 
     // lanes finish their steps at different iterations runs one sample path, not a second one in
     // the branch of the finishing lanes; each lane's sequence of operations is unchanged.
     bool emit_next = false, conv_out = false;
+    MidRange<RN> mr;
     while (true) {
         const float4 fe = sample(pos.x, pos.y, pos.z);
         bool emit = emit_next;
         emit_next = false;
         if (!emit) {
-            f3 f = mk3(fe.x, fe.y, fe.z);
             const f3 dp = mk3(pos.x - tip.x, pos.y - tip.y, pos.z - tip.z);
+            f3 f = mk3(fe.x, fe.y, fe.z);
             if constexpr (IDF) {
-                const f3 ft = tipForce(dp, p.k, p.d0);
+                const f3 ft = tipForce<RN>(dp, p.k, p.d0, mr);
                 f = mk3(f.x + ft.x, f.y + ft.y, f.z + ft.z);
                 f.z = f.z + p.surf;
             } else {
-                const f3 ft = rotMatT(tipForce(rotMat(dp, A, B, C), p.k, p.d0), A, B, C);
+                const f3 ft = rotMatT(tipForce<RN>(rotMat(dp, A, B, C), p.k, p.d0, mr), A, B, C);
                 f = mk3(f.x + ft.x, f.y + ft.y, f.z + ft.z);
                 f = mk3(f.x + fsurf.x, f.y + fsurf.y, f.z + fsurf.z);
             }
@@ -386,7 +464,7 @@ __device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, 
             if (p.check_before && ff < p.f2conv) {
                 conv = done = true;
             } else {
-                v = integrate(p.damped, f, v, dt, damp, dtmin, dtmax, damp0);
+                v = integrate<RN>(p.damped, f, v, dt, damp, dtmin, dtmax, damp0, mr);
                 v = mk3(v.x + f.x * dt, v.y + f.y * dt, v.z + f.z * dt);
                 pos = mk3(pos.x + v.x * dt, pos.y + v.y * dt, pos.z + v.z * dt);
                 if (!p.check_before && ff < p.f2conv) conv = done = true;
@@ -427,16 +505,13 @@ __device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, 
             ++pend;
             const bool last = iz + 1 >= p.nz;
             if (STAGE && LDSST && (last || (reinterpret_cast<uintptr_t>(FEs + o + 1) & 63) == 0)) {
-                float4* dst = FEs + o - (pend - 1);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k < pend) dst[k] = stage[k * 64];
-                if (PPs) {
-                    float4* dq = PPs + o - (pend - 1);
+                auto run = [&](float4* dst, const float4* src) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        if (k < pend) dq[k] = stage[(4 + k) * 64];
-                }
+                        if (k < pend) dst[k] = src[k * 64];
+                };
+                run(FEs + o - (pend - 1), stage);
+                if (PPs) run(PPs + o - (pend - 1), stage + 4 * 64);
                 pend = 0;
             } else if (STAGE && !LDSST && (last || (reinterpret_cast<uintptr_t>(FEs + o + 1) & 63) == 0)) {
                 if (G == 1) {
@@ -459,9 +534,25 @@ __device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, 
             }
             v = mk3(0.f, 0.f, 0.f);
             it = 0;
-            if (++iz >= p.nz) break;
+            if (++iz >= p.nz || mr.out()) break;
         }
     }
+    return !mr.out();
+}
+template <int G, class SAMPLE, bool STAGE = true, bool IDF = false, bool LDSST = false>
+__device__ __forceinline__ void relax_tilted_lane_src(SAMPLE& sample, f3 start, const TiltArgs& p,
+                                                      float4* __restrict__ FEs, float4* __restrict__ PPs,
+                                                      int sub = 0, const DfOut* dfo = nullptr,
+                                                      float* __restrict__ dfrow = nullptr,
+                                                      float* __restrict__ fz_lds = nullptr,
+                                                      float4* __restrict__ stage = nullptr) {
+    sample.begin();
+    if (!p.short_ops || !relax_tilted_column<true, G, SAMPLE, STAGE, IDF, LDSST>(sample, start, p, FEs, PPs, sub,
+                                                                                 fz_lds, stage)) {
+        sample.begin();
+        relax_tilted_column<false, G, SAMPLE, STAGE, IDF, LDSST>(sample, start, p, FEs, PPs, sub, fz_lds, stage);
+    }
+    sample.end();
     if (dfo && fz_lds) {         // the lane's own copy of the column; the group splits the outputs
         for (int j = sub; j < dfo->nout; j += G) {
             const int s0 = dfo->start[j];
@@ -499,11 +590,9 @@ __device__ __forceinline__ void relax_tilted_lane(const GridDev& g, f3 start, co
                                                   const DfOut* dfo = nullptr, float* __restrict__ dfrow = nullptr,
                                                   float* __restrict__ fz_lds = nullptr,
                                                   float4* __restrict__ stage = nullptr) {
-    Cell cell;
-    cell.reset();
-    auto smp = [&](float x, float y, float z) { return sample<FAST>(g, cell, x, y, z); };
-    relax_tilted_lane_src<1, decltype(smp), STAGE, FAST, LDSST>(smp, start, p, FEs, PPs, 0, dfo, dfrow, fz_lds,
-                                                                stage);
+    GridSample<1, FAST> smp{g, 0};
+    relax_tilted_lane_src<1, GridSample<1, FAST>, STAGE, FAST, LDSST>(smp, start, p, FEs, PPs, 0, dfo, dfrow, fz_lds,
+                                                                      stage);
 }
 
 }  // namespace rc
