@@ -20,6 +20,8 @@
 // (one sincospi per G and column, shared by kVz planes) and
 //   E = t0 + sum_G Re(T_G p),  F = (sum_G Gx Im(T_G p), sum_G Gy Im(T_G p), -t0' - sum_G Re(T'_G p)),
 // i.e. F = -grad E.  A workgroup stages the tables of its planes through LDS in chunks of G.
+#include <algorithm>
+
 #include "ppm_common.hpp"
 
 namespace ppm {
@@ -313,6 +315,258 @@ __global__ __launch_bounds__(256) void k_ewald_grid(const float4* __restrict__ t
     }
 }
 
+// Grids whose first axis runs along the lattice vector a (b2.dA = 0): the phase of G = h b1 + k b2 then moves
+// along a grid row with h alone, e^{i G.(p0 + ib dB + ia dA)} = e^{i G.(p0 + ib dB)} u^(h ia), so that a row's
+// sum over G is taken in two parts: the G of one h join into the row's coefficient of u^(h ia), and a voxel sums
+// one term per distinct h (41 instead of 462 for the 8 x 8 slab at n_harm 40).  The second part is a matrix
+// product, (row, component) x (h; cos, sin) x (ia), on the FP32 matrix cores:
+//   * v_mfma_f32_32x32x2_f32 with the k pair = (cos, sin) of one h; its D registers hold 4 consecutive m in a
+//     lane, so m = 4 row + component makes them the float4 of a voxel, and n = ia makes a wave's store two runs
+//     of 512 bytes;
+//   * a workgroup keeps the coefficients of 8 rows (one plane, successive ib) in LDS, its waves walk along ia in pairs of
+//     tiles of 32, which share each coefficient read;
+//   * u^(h ia) = u^(h 32 t) u^(h j): the j factors are in LDS, each wave makes the factors of its pair of tiles there,
+//     a lane for each h and tile (VALU instructions and FP32 MFMAs did not overlap in this kernel, so both factors
+//     come from LDS in the form that a lane multiplies: 2 instructions for a phase); every phase is reduced to a fraction of a turn in FP64 before it is rounded;
+//   * an h is left out of a workgroup's product if that moves no sum by more than 1/16 of what rounding it does: its
+//     coefficient is below 2^-28 / (number of h) of the sum of all coefficients, in every row and component.  The
+//     terms fall off as e^{-|G| z}, and at n_harm 40 two thirds of them end there.
+// Bound by its instructions, FP32 MFMAs (64 cycles for each h and 32 x 8 voxels) and VALU in turn, for many h, and by
+// the stores for few.  902 x 902 x 120 voxels: 462 kept G in 41 h 10.04 -> 0.63 ms (of it MFMA 0.28, and with one h
+// 0.35), 30 kept G in 6 h 1.04 -> 0.34 ms (4.5 TB/s of stores).
+using f32x16 = float __attribute__((ext_vector_type(16)));
+constexpr int kRowTile = 8;                  // rows of a workgroup
+constexpr int kRowWaves = 4;
+constexpr int kMaxH = 64;                    // distinct h: one per lane for the tile factors
+
+struct RowArgs {
+    int n_g, na, nb, nz, n_harm, tiles, split;      // tiles of 32 ia in all and per workgroup
+    double p0[2], dB[2], b1[2], b2[2];
+    double turn;                                    // b1.dA / 2 pi
+    int accumulate;
+};
+
+// LDS of a workgroup: coefficients [piece, then h][64] (at most two pieces for an h, on average); the j factors [h][32], before them the factors of the coefficients
+// (per row: k: 2 n_harm + 1, h: n_harm + 1) and the k of the kept G; the tile factors [wave][h][tile][3]; the
+// distinct h, where each begins, the pieces.
+inline __host__ __device__ size_t row_mid(int n_harm) {
+    const size_t coef = (size_t)(3 * n_harm + 2) * kRowTile * 8 + (size_t)2 * n_harm * (n_harm + 1);
+    const size_t off = (size_t)(n_harm + 1) * 256, red = (kRowWaves * 64 + 2 * kRowWaves) * 4;
+    return (std::max(std::max(coef, off), red) + 15) & ~size_t(15);
+}
+inline size_t row_lds(int n_harm) { return (size_t)(n_harm + 1) * 512 + row_mid(n_harm) + (size_t)(n_harm + 1) * kRowWaves * 24 +
+                                               (5 * kMaxH + 4) * 4; }
+
+// (cos, sin) of f turns; f is reduced in FP64.
+__device__ __forceinline__ float2 turns(double f) {
+    float2 p;
+    sincospif(2.0f * (float)(f - rint(f)), &p.y, &p.x);
+    return p;
+}
+
+__global__ __launch_bounds__(kRowWaves * 64, 4) void k_ewald_rows(const float4* __restrict__ tab, const float2* __restrict__ zt,
+                                                       const float4* __restrict__ ginfo, const int* __restrict__ cntp,
+                                                       RowArgs a, float4* __restrict__ out) {
+    constexpr int kThreads = kRowWaves * 64;
+    extern __shared__ float4 s_row[];
+    char* mid = reinterpret_cast<char*>(s_row) + (size_t)(a.n_harm + 1) * 512;
+    float4* sA = s_row;
+    float2* sOff = reinterpret_cast<float2*>(mid);
+    float2* sP = sOff;                        // of each row e^{i k t2} at k + n_harm, then e^{i h t1}
+    const int np = 3 * a.n_harm + 2;
+    signed char* sGk = reinterpret_cast<signed char*>(sP + np * kRowTile);
+    float* sTile = reinterpret_cast<float*>(mid + row_mid(a.n_harm));
+    int* sH = reinterpret_cast<int*>(sTile + (a.n_harm + 1) * kRowWaves * 6);
+    int* sFirst = sH + kMaxH;                                         // [kMaxH + 1]
+    int* sPiece = sFirst + kMaxH + 1;         // [kMaxH + 1]: the first piece of each h
+    unsigned short* sOf = reinterpret_cast<unsigned short*>(sPiece + kMaxH + 1);      // [2 kMaxH]: h | part << 6 of a piece
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+    const int ib0 = (int)blockIdx.x * kRowTile, iz = blockIdx.y;
+    const int cnt = min(max(cntp[0], 0), min(a.n_g, 2 * a.n_harm * (a.n_harm + 1)));
+
+    // the kept G (h outermost): their k, the distinct h in order and where each begins
+    if (tid < kMaxH) sFirst[tid] = -1;
+    __syncthreads();
+    for (int c = tid; c < cnt; c += kThreads) {
+        const float4 G = ginfo[c];
+        sGk[c] = (signed char)(int)G.w;
+        if (c == 0 || ginfo[c - 1].z != G.z) sFirst[(int)G.z & (kMaxH - 1)] = c;
+    }
+    {
+        const int row = tid >> 5, ib = ib0 + row;
+        const double x = a.p0[0] + ib * a.dB[0], y = a.p0[1] + ib * a.dB[1];
+        double t1 = (a.b1[0] * x + a.b1[1] * y) * (0.5 / kPi), t2 = (a.b2[0] * x + a.b2[1] * y) * (0.5 / kPi);
+        t1 -= floor(t1);
+        t2 -= floor(t2);
+        for (int j = tid & 31; j < np; j += 32)
+            sP[row * np + j] = turns(j <= 2 * a.n_harm ? (j - a.n_harm) * t2 : (j - 2 * a.n_harm - 1) * t1);
+    }
+    __syncthreads();
+    const int mine = sFirst[lane];
+    const unsigned long long have = __ballot(mine >= 0);
+    int nh = __popcll(have);
+    __syncthreads();
+    if (wave == 0 && mine >= 0) {
+        const int q = __popcll(have & ((1ull << lane) - 1));
+        sH[q] = lane;
+        sFirst[q] = mine;
+    }
+    if (tid == 0) sFirst[nh] = cnt;
+    __syncthreads();
+    // pieces: an h with many k is summed by several lanes (the kept k of an h range from 6 to 80 in the 8 x 8 slab)
+    const int len = 8 * max(1, (cnt + 8 * a.n_harm + 7) / (8 * a.n_harm + 8));
+    int end = lane < nh ? (sFirst[lane + 1] - sFirst[lane] + len - 1) / len : 0;
+    const int parts = end;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(end, o);
+        if (lane >= o) end += v;
+    }
+    const int npiece = __builtin_amdgcn_readfirstlane(__shfl(end, 63));
+    if (wave == 0) {
+        sPiece[lane] = end - parts;
+        if (lane == 63) sPiece[64] = end;
+        for (int u = 0; u < parts; ++u) sOf[end - parts + u] = (unsigned short)(lane | u << 6);
+    }
+    __syncthreads();
+
+    // Coefficients of (row, piece), 32 lanes to a row.  A = sum_k T e^{i k t2}, B = sum_k k T e^{i k t2}, Z the sum of
+    // T', each times e^{i h t1}: E = Re(A p), F = (Im((h b1x A + b2x B) p), Im((h b1y A + b2y B) p), -Re(Z p)).
+    {
+        constexpr int U = 8;
+        const int row = tid >> 5;
+        const float2 *sK = sP + row * np, *sE = sK + 2 * a.n_harm + 1;
+        const float4* T = tab + (size_t)iz * a.n_g;
+        const float b1x = (float)a.b1[0], b1y = (float)a.b1[1], b2x = (float)a.b2[0], b2y = (float)a.b2[1];
+        for (int u = tid & 31; u < npiece; u += 32) {
+            const int q = sOf[u] & 63, j0 = sFirst[q] + (sOf[u] >> 6) * len, e = min(j0 + len, sFirst[q + 1]);
+            float Ar = 0.f, Ai = 0.f, Br = 0.f, Bi = 0.f, Zr = 0.f, Zi = 0.f;
+            for (int j = j0; j < e; j += U) {
+                float4 t[U];
+#pragma unroll
+                for (int w = 0; w < U; ++w) t[w] = T[min(j + w, e - 1)];
+#pragma unroll
+                for (int w = 0; w < U; ++w) {
+                    const int k = sGk[min(j + w, e - 1)];
+                    float2 p = sK[k + a.n_harm];
+                    if (j + w >= e) p = make_float2(0.f, 0.f);
+                    const float re = fmaf(t[w].x, p.x, -(t[w].y * p.y)), im = fmaf(t[w].x, p.y, t[w].y * p.x);
+                    Ar += re;
+                    Ai += im;
+                    Br = fmaf((float)k, re, Br);
+                    Bi = fmaf((float)k, im, Bi);
+                    Zr = fmaf(t[w].z, p.x, fmaf(-t[w].w, p.y, Zr));
+                    Zi = fmaf(t[w].z, p.y, fmaf(t[w].w, p.x, Zi));
+                }
+            }
+            const float h = (float)sH[q];
+            const float2 w = sE[sH[q]];
+            auto turn = [&](float& r, float& i) {
+                const float x = fmaf(r, w.x, -(i * w.y));
+                i = fmaf(r, w.y, i * w.x);
+                r = x;
+            };
+            turn(Ar, Ai);
+            turn(Br, Bi);
+            turn(Zr, Zi);
+            const float gx = h * b1x, gy = h * b1y;
+            float4* dst = sA + u * 16 + row;
+            dst[0] = make_float4(fmaf(gx, Ai, b2x * Bi), fmaf(gy, Ai, b2y * Bi), -Zr, Ar);        // cos
+            dst[8] = make_float4(fmaf(gx, Ar, b2x * Br), fmaf(gy, Ar, b2y * Br), Zi, -Ai);        // sin
+        }
+    }
+    __syncthreads();
+    // leave out what is below the rounding of the sums; wave w looks at h = w, w + 4, ...
+    {
+        constexpr int N = kMaxH / kRowWaves;
+        float* red = reinterpret_cast<float*>(mid);                   // [kRowWaves][64]
+        unsigned long long* keeps = reinterpret_cast<unsigned long long*>(red + kRowWaves * 64);
+        float* sAf = reinterpret_cast<float*>(sA);
+        float v[N], sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int q = i * kRowWaves + wave;
+            v[i] = 0.f;
+            if (q < nh)
+                for (int u = sPiece[q]; u < sPiece[q + 1]; ++u) v[i] += sAf[u * 64 + lane];
+            sum += fabsf(v[i]);
+        }
+        red[wave * 64 + lane] = sum;
+        const int hq = lane < nh ? sH[lane] : 0;
+        __syncthreads();
+        sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) sum += red[w * 64 + lane] + red[w * 64 + (lane ^ 32)];
+        const float least = sum * (0x1p-28f / (float)max(nh, 1));
+        unsigned long long keep = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const bool big = !(fabsf(v[i]) < least) && v[i] != 0.f;   // not finite: kept
+            if (__ballot(big)) keep |= 1ull << (i * kRowWaves + wave);
+        }
+        if (lane == 0) keeps[wave] = keep;
+        __syncthreads();
+        keep = 0;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) keep |= keeps[w];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int q = i * kRowWaves + wave;
+            if (keep >> q & 1) sAf[__popcll(keep & ((1ull << q) - 1)) * 64 + lane] = v[i];
+        }
+        if (wave == 0 && (keep >> lane & 1)) sH[__popcll(keep & ((1ull << lane) - 1))] = hq;
+        nh = __builtin_amdgcn_readfirstlane(__popcll(keep));
+    }
+    __syncthreads();
+    for (int u = tid; u < nh * 32; u += kThreads) sOff[u] = turns(a.turn * sH[u >> 5] * (u & 31));
+    __syncthreads();
+
+    const int t1 = min(((int)blockIdx.z + 1) * a.split, a.tiles), t0 = (int)blockIdx.z * a.split + 2 * wave;
+    const float2 z0 = zt[iz];
+    const float* pa = reinterpret_cast<const float*>(sA) + lane;
+    const float2* po = sOff + (lane & 31);
+    // of tile factor e^{if} the triple (-sin f, cos f, sin f): the lower half of the wave multiplies (cos f, -sin f)
+    // into (cos g, sin g) for cos(f + g), the upper (sin f, cos f) for sin(f + g)
+    float* tile = sTile + wave * (a.n_harm + 1) * 6;
+    const float* pt = tile + half;
+    const int row0 = ib0 + half;
+    float4* dst = out + ((size_t)iz * a.nb + row0) * a.na + (lane & 31);
+    for (int t = t0; t < t1; t += 2 * kRowWaves) {
+        for (int u = lane; u < 2 * nh; u += 64) {
+            const float2 f = turns(a.turn * sH[u >> 1] * (32.0 * (t + (u & 1))));
+            tile[3 * u] = -f.y;
+            tile[3 * u + 1] = f.x;
+            tile[3 * u + 2] = f.y;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");      // one wave: its LDS operations stay in order
+        f32x16 d0 = {0}, d1 = {0};
+#pragma unroll 4
+        for (int h = 0; h < nh; ++h) {
+            const float co = pa[h * 64];
+            const float2 o = po[h * 32];
+            const float* f = pt + h * 6;
+            d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(co, fmaf(f[0], o.y, f[1] * o.x), d0, 0, 0, 0);
+            d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(co, fmaf(f[3], o.y, f[4] * o.x), d1, 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        auto store = [&](const f32x16& d, int tile) {
+            if (tile >= t1 || tile * 32 + (lane & 31) >= a.na) return;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (row0 + 2 * q >= a.nb) break;
+                float4* o = dst + (tile * 32 + (size_t)(2 * q) * a.na);
+                float4 v = make_float4(d[4 * q], d[4 * q + 1], d[4 * q + 2] - z0.y, d[4 * q + 3] + z0.x);
+                if (a.accumulate) {
+                    const float4 old = *o;
+                    v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+                }
+                *o = v;
+            }
+        };
+        store(d0, t);
+        store(d1, t + 1);
+    }
+}
+
 // phi at points (n,4) = (x,y,z,-), C included, FP64 accumulation over the kept G.
 // mode 0: the full form (eval_potential_full, kernels/surface.cl:1172-1246), any z;
 // mode 1: the vacuum form (eval_potential_vacuum, kernels/surface.cl:1103-1157): no G = 0 term,
@@ -485,6 +739,31 @@ int launch_ewald_tip_grid(const void* system, int n_layers, int n_harm, const do
     hipLaunchKernelGGL(k_plane_tables, dim3(blocks_for((long long)gs.nz * (g.n_g + 1))), dim3(256), 0, stream, s, g,
                        gs.nz, (double)gs.p0[2], (double)gs.dC[2], qs, qz, tab, zt);
     if (int r = check_launch("ewald_tables")) return r;
+    // The rows' form needs the first grid axis along a: b2.dA so small that the phase of no G moves by more than
+    // 2^-27 of a turn over a row from it (FP32 rounds phases at 2^-25); and one lane per h.  It is the faster one
+    // at every size tried, from 64 x 64 x 16 voxels with 30 G on.
+    const double skew = fabs(g.b2[0] * gs.dA[0] + g.b2[1] * gs.dA[1]) * (0.5 / kPi) * n_harm * gs.nx;
+    if (skew <= 0x1p-27 && n_harm < kMaxH && gs.nz <= 65535) {
+        RowArgs ra{};
+        ra.n_g = g.n_g; ra.na = gs.nx; ra.nb = gs.ny; ra.nz = gs.nz; ra.n_harm = n_harm;
+        ra.accumulate = accumulate;
+        for (int q = 0; q < 2; ++q) {
+            ra.p0[q] = gs.p0[q]; ra.dB[q] = gs.dB[q]; ra.b1[q] = g.b1[q]; ra.b2[q] = g.b2[q];
+        }
+        ra.turn = (g.b1[0] * gs.dA[0] + g.b1[1] * gs.dA[1]) * (0.5 / kPi);
+        ra.tiles = (gs.nx + 31) / 32;
+        const int chunks = (gs.ny + kRowTile - 1) / kRowTile;
+        // the walk along ia is cut, down to one pair of tiles for each wave, while the launch has fewer workgroups than
+        // the card holds (4 per compute unit); each cut takes the coefficients again
+        const long long rows = (long long)gs.nz * chunks;
+        const int cuts = (int)std::min<long long>((ra.tiles + 2 * kRowWaves - 1) / (2 * kRowWaves),
+                                                  std::max<long long>(1, 1024 / rows));
+        ra.split = (ra.tiles + cuts - 1) / cuts;
+        const dim3 grd((unsigned)chunks, (unsigned)gs.nz, (unsigned)((ra.tiles + ra.split - 1) / ra.split));
+        hipLaunchKernelGGL(k_ewald_rows, grd, dim3(kRowWaves * 64), row_lds(n_harm), stream, tab, zt, s.ginfo, s.cnt, ra,
+                           reinterpret_cast<float4*>(grid));
+        return check_launch("ewald_rows");
+    }
     const dim3 grd(blocks_for((long long)gs.nx * gs.ny), (unsigned)((gs.nz + kVz - 1) / kVz));
     hipLaunchKernelGGL(k_ewald_grid, grd, dim3(256), 0, stream, tab, zt, s.ginfo, s.cnt, g.n_g, gs.nx, gs.ny, gs.nz,
                        gs.p0[0], gs.p0[1], gs.dA[0], gs.dA[1], gs.dB[0], gs.dB[1], (float)g.b1[0], (float)g.b1[1],
