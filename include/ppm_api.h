@@ -127,7 +127,7 @@ typedef struct PpmBatchParams {
     PpmRelaxCtl ctl;
 } PpmBatchParams;
 
-#define PPM_BATCH_FUSED       0   /* grid tiles and relaxation blocks from one work queue */
+#define PPM_BATCH_FUSED       0   /* the grid launch and then the relaxation launch, in one call */
 #define PPM_BATCH_GRID_ONLY   1
 #define PPM_BATCH_RELAX_ONLY  2
 
@@ -502,13 +502,14 @@ int ppm_batch_grid_items(const PpmMolDesc* mol, const PpmBatchParams* params);
 /* Batched forward (no reference counterpart: the reference runs one image at a time through
  * make_forcefield / run_scan / compute_df, spammm/SPM/AFM.py:897-1010, :3048-3089).
  * Runs grid projection, relaxed scan (relaxStrokesTilted semantics) and the df operator of
- * every molecule described by `mols` (device array of params->nmol PpmMolDesc) in one
- * persistent launch of `workers` workgroups.
+ * every molecule described by `mols` (device array of params->nmol PpmMolDesc) in two
+ * persistent launches of `workers` workgroups, one over the grid tiles and one over the
+ * relaxation blocks.
  *   atoms / cpar: concatenated rows of all molecules (PpmMolDesc.atom_off);
  *   grids: stored z windows of all grids; FEs, PPs (PPs may be NULL): (n_pix_total, nz, 4);
  *   df (may be NULL): (n_pix_total, df_nz_out), operator dfW (df_nz_out*df_taps), dfStart;
  *   workspace: >= ppm_batch_workspace_size(nmol) bytes; after the call workspace int[1] is
- *     the error word (bit 1: a wait hit its spin limit) and ints [4+nmol, 4+2*nmol) are
+ *     the error word (bit 1: a molecule was relaxed before all its tiles were projected) and ints [4+nmol, 4+2*nmol) are
  *     per-molecule flags (nonzero: a probe left the stored z window — recompute that molecule
  *     with the whole grid);
  *   reset: 1 = clear queue, counters and flags first; 2 = clear the queue head only (second
@@ -532,7 +533,7 @@ int ppm_batch_forward(const PpmMolDesc* mols, const PpmBatchParams* params,
  * the process ends; its address is looked up on the first call on each device, which must be the
  * current device) instead of a caller workspace; params->nmol <= PPM_BATCH_NOALLOC_MAX_MOL.
  *   status: device int[1 + nmol], written after the launch: status[0] = error word (bit 1: a
- *     wait hit its spin limit), status[1 + m] = window flag of molecule m (nonzero: recompute m
+ *     molecule was relaxed before all its tiles were projected), status[1 + m] = window flag of molecule m (nonzero: recompute m
  *     with the whole grid);
  *   reset: 1 (clear queue, counters and flags first) or 2 (clear the queue head only: the
  *     RELAX_ONLY launch that follows a GRID_ONLY launch); 0 is rejected.

@@ -1,10 +1,9 @@
 """Autotuner of the batched forward's launch shape.
 
 Candidates: grid voxels per thread along z (4, 8), the pixel tile of a wavefront (16x4, 8x8,
-4x16 pixels), persistent workgroups per compute unit (2, 3, 4), the schedule (one fused
-launch, or a grid launch followed by a relaxation launch) and, for the fused launch, the queue
-lag (0: each molecule's relaxation blocks right after its tiles; k: after the tiles of molecule
-m + k).  Each candidate runs the real batch
+4x16 pixels), persistent workgroups per compute unit (2, 3, 4), the schedule (one library call,
+or one for the grid launch and one for the relaxation launch) and the queue order (lag 0: each
+molecule's relaxation blocks right after its tiles; k: after the tiles of molecule m + k).  Each candidate runs the real batch
 (or a prefix of it) and is timed with HIP events on the launch stream; every candidate's df
 must equal the first candidate's bit for bit (they compute the same arithmetic, only the
 work decomposition differs).  The winner is cached in a JSON file keyed by device name and a
@@ -94,11 +93,11 @@ def tune(batch: BatchForward, candidates=None, reps: int = 2, use_cache: bool = 
     for vals in itertools.product(*(cand[k] for k in keys)):
         cfg = LaunchConfig(**dict(zip(keys, vals)))
         if cfg.schedule == "two_phase" and cfg.lag:
-            continue        # the lag orders fused work only (two phases separate the kinds anyway)
+            continue        # two calls at one lag are enough
         ms = time_config(batch, cfg, reps)
         err, _ = batch.status()
         if err:
-            raise RuntimeError(f"autotune: launch {cfg.key()} reported a wait timeout")
+            raise RuntimeError(f"autotune: launch {cfg.key()} reported unfinished tiles")
         out = batch.df.clone() if batch.df is not None else batch.FEs.clone()
         if ref is None:
             ref = out
@@ -118,8 +117,7 @@ def tune(batch: BatchForward, candidates=None, reps: int = 2, use_cache: bool = 
 def refine(batch: BatchForward, cfg: LaunchConfig, lags=(32, 64), reps: int = 2, log=None):
     """The tuned shape ``cfg`` checked on the whole ``batch``: the same vz, tile and workgroups per
     CU as two-phase and as fused with each queue lag in ``lags`` (lags longer than the tuning
-    sample's molecule count; a relaxation block then finds its tiles done instead of waiting), each
-    timed on the whole batch; returns (the fastest, {key: ms}).  Every variant must give the first
+    sample's molecule count), each timed on the whole batch; returns (the fastest, {key: ms}).  Every variant must give the first
     one's results bit for bit."""
     import torch
     variants = [cfg, LaunchConfig(cfg.vz, cfg.tile_w, cfg.workers_per_cu, "two_phase", 0)]
@@ -134,7 +132,7 @@ def refine(batch: BatchForward, cfg: LaunchConfig, lags=(32, 64), reps: int = 2,
         ms = time_config(batch, v, reps)
         err, _ = batch.status()
         if err:
-            raise RuntimeError(f"autotune: launch {v.key()} reported a wait timeout")
+            raise RuntimeError(f"autotune: launch {v.key()} reported unfinished tiles")
         out = batch.df.clone() if batch.df is not None else batch.FEs.clone()
         if ref is None:
             ref = out

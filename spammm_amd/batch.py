@@ -1,4 +1,4 @@
-"""Batched forward: hundreds of molecules through grid -> relax -> df in one persistent launch.
+"""Batched forward: hundreds of molecules through grid -> relax -> df in two persistent launches.
 
 ``BatchForward`` packs molecules of uneven atom counts and cell sizes into one set of device
 buffers and one descriptor array (``PpmMolDesc``, include/ppm_api.h), then runs
@@ -6,7 +6,7 @@ buffers and one descriptor array (``PpmMolDesc``, include/ppm_api.h), then runs
 atomic work queue (molecule by molecule), each lane relaxes one pixel through its z descent
 and applies the df operator to its own Fz column.  The launch can be captured in a hipGraph
 (``capture``/``replay``).  Launch shape (voxels per thread, pixel tile per wavefront,
-workgroups per CU, fused or two-launch schedule) is chosen by ``spammm_amd.autotune``.
+workgroups per CU, one library call or two) is chosen by ``spammm_amd.autotune``.
 
 Only the z planes a probe can reach are projected: the planes covering the probe rest heights
 of the scan (tip anchor + dpos0) widened by ``z_margin`` A below and above (default 0.3, 0.5:
@@ -52,7 +52,7 @@ class LaunchConfig:
     vz: int = 8                 # grid tile size (8 large, 4 small)
     tile_w: int = 8             # pixels along iy of a wavefront's 64-pixel tile
     workers_per_cu: int = 3     # persistent workgroups per compute unit
-    schedule: str = "fused"     # "fused" (one launch) or "two_phase" (grid launch, then relax launch)
+    schedule: str = "fused"     # "fused" (one call: grid launch, relax launch) or "two_phase" (a call for each)
     lag: int = 0                # queue order: the tiles of molecule m + lag come before the blocks of m
 
     def key(self):

@@ -1,17 +1,17 @@
 // ppm_batch.hip — batched forward: many molecules (uneven atom counts, cell sizes and grid
-// shapes) through grid projection -> relaxed scan -> df in ONE persistent launch.
+// shapes) through grid projection -> relaxed scan -> df in two persistent launches.
 //
-// Work items: for each molecule m its grid tiles (256 columns x vz planes of the stored z window)
-// and its relaxation blocks (4 wavefronts x 64 pixels; each lane relaxes one pixel through all
-// z-steps and then applies the df operator to its own Fz column), as two queue segments; the host
-// orders the segments (by default each molecule's blocks right after its tiles; with a lag k the
-// tiles of m + k come before the blocks of m, so a block rarely waits for its tiles).
-// Persistent workgroups take items from an atomic counter.  A relaxation block of m waits (with
-// a bounded spin) until every grid tile of m has been published: the tile's stores are released
-// at agent scope before the per-molecule counter is incremented, and the waiting workgroup
-// acquires at agent scope before it reads the grid, so the data crosses XCD L2 caches correctly.
-// Items are taken in increasing order, so a waited-for tile has always been taken by a running
-// workgroup: the wait ends.  Every workgroup leaves the loop when the queue is exhausted.
+// Work items: for each molecule m its grid tiles (256 columns x vz planes of the stored z window, or
+// shares of the far form's blocks) and its relaxation blocks (4 wavefronts x 64 pixels; each lane
+// relaxes one pixel through all z-steps and then applies the df operator to its own Fz column), as two
+// queue segments.  Persistent workgroups take items from an atomic counter, in a grid launch that
+// passes over the blocks and a relaxation launch that passes over the tiles.
+//
+// Why two launches: tiles and blocks want different workgroups.  The far form's LDS (53 KB) and
+// registers hold 3 workgroups on a compute unit, the relaxation alone 4, without spilling; and in one
+// launch a block waited for the molecule's last tiles while it held its place.  Batches of 1 | 24 | 384
+// molecules (U{10..150} atoms): one launch 2.43 | 10.5 | 148 ms (8.7 | 125 with the tiles taken far
+// ahead), two 2.12 | 7.1 | 101 ms.
 //
 // The grid and relaxation arithmetic is the device code of the plain kernels
 // (ppm_grid_core.hpp, ppm_relax_core.hpp), so each molecule's results equal the plain path's
@@ -29,12 +29,9 @@ namespace {
 using gc::GridArgs;
 using gc::Site;
 
-
-constexpr int kSpinLimit = 1 << 20;     // polls (~1 us each with the sleep): a bound of about a second
-
 struct Queue {           // device workspace, zeroed by k_batch_reset
     int head;            // next work item
-    int error;           // bit 1: a wait hit the spin limit
+    int error;           // bit 1: a relaxed molecule's tiles were not all projected
     int pad[2];
     // followed by: int done[nmol]; int flag[nmol];
 };
@@ -192,110 +189,97 @@ __device__ void do_relax_item(const PpmMolDesc& d, const PpmBatchParams& P, int 
         rc::relax_tilted_lane<false, false>(g, start, t, FEs + o, pp, df ? &dfo : nullptr, dr);
 }
 
-// OFFQ: the tip has charge sites at a nonzero z offset (compiled out when it has none).  GRID = false:
-// a launch of relaxation blocks only, without the grid code's registers and LDS (53 KB: 3 workgroups per
-// compute unit), which leaves the relaxation more waves.
-template <int MODEL, bool HASQ0, int V, bool OFFQ, bool GRID>
-__global__ __launch_bounds__(256, GRID ? 3 : 4) void k_batch(const PpmMolDesc* __restrict__ mols, PpmBatchParams P,
-                                               const float4* __restrict__ atoms, const float* __restrict__ cpar,
-                                               float4* __restrict__ grids, float4* __restrict__ FEs,
-                                               float4* __restrict__ PPs, float* __restrict__ df,
-                                               const float* __restrict__ dfW, const int* __restrict__ dfStart,
-                                               Queue* q) {
+// The next work item: false when the queue is exhausted; else its molecule m and `local`, its number among
+// the molecule's tiles and then blocks.  done_m: molecule whose tile the workgroup finished before (-1:
+// none).  Thread 0 counts it here, in the same thread-0 section as the dequeue: a thread-0-only section at
+// the END of the caller's loop body would be merged by the compiler with the one at the top into a
+// divergent inner loop whose other lanes re-read the stale item after the barrier and never leave it.
+__device__ __forceinline__ bool take_item(const PpmMolDesc* mols, const PpmBatchParams& P, Queue* q, int done_m, int& m,
+                                          int& local) {
     __shared__ int s_item, s_mol, s_local;
-    int* done = q_done(q);
-    int* flags = q_flag(q, P.nmol);
-    // Molecule whose grid tile this workgroup finished in the previous iteration (-1: none).
-    // Thread 0 publishes it at the top of the next iteration, in the same thread-0 section
-    // as the dequeue: a thread-0-only section at the END of the loop body would be merged by
-    // the compiler with the one at the top into a divergent inner loop whose other lanes
-    // re-read the stale item after the barrier and never leave it.
-    int signal_m = -1;
-    while (true) {
-        if (threadIdx.x == 0) {
-            if (signal_m >= 0) __hip_atomic_fetch_add(&done[signal_m], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            int item = atomicAdd(&q->head, 1);
-            int m = -1, local = 0;
-            if (item < P.nitems) {
-                int lo = 0, hi = P.nmol - 1;            // last molecule with item_off <= item
+    if (threadIdx.x == 0) {
+        if (done_m >= 0) atomicAdd(&q_done(q)[done_m], 1);
+        const int item = atomicAdd(&q->head, 1);
+        int mol = -1, loc = 0;
+        if (item < P.nitems) {
+            int lo = 0, hi = P.nmol - 1;            // last molecule with item_off <= item
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (mols[mid].item_off <= item) lo = mid; else hi = mid - 1;
+            }
+            if (item < mols[lo].item_off + mols[lo].n_grid_items) {
+                mol = lo;
+                loc = item - mols[lo].item_off;
+            } else {                                // a relaxation block: last molecule whose
+                lo = 0;                             // relaxation segment starts at or before item
+                hi = P.nmol - 1;
                 while (lo < hi) {
                     const int mid = (lo + hi + 1) >> 1;
-                    if (mols[mid].item_off <= item) lo = mid; else hi = mid - 1;
+                    if (relax_start(mols[mid]) <= item) lo = mid; else hi = mid - 1;
                 }
-                if (item < mols[lo].item_off + mols[lo].n_grid_items) {
-                    m = lo;
-                    local = item - mols[lo].item_off;
-                } else {                                // a relaxation block: last molecule whose
-                    lo = 0;                             // relaxation segment starts at or before item
-                    hi = P.nmol - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (relax_start(mols[mid]) <= item) lo = mid; else hi = mid - 1;
-                    }
-                    m = lo;
-                    local = mols[lo].n_grid_items + (item - relax_start(mols[lo]));
-                }
+                mol = lo;
+                loc = mols[lo].n_grid_items + (item - relax_start(mols[lo]));
             }
-            s_item = item;
-            s_mol = m;
-            s_local = local;
         }
-        __syncthreads();
-        const int item = __builtin_amdgcn_readfirstlane(s_item), m = __builtin_amdgcn_readfirstlane(s_mol);
-        const int local = __builtin_amdgcn_readfirstlane(s_local);
-        __syncthreads();
-        if (item >= P.nitems) break;
+        s_item = item;
+        s_mol = mol;
+        s_local = loc;
+    }
+    __syncthreads();
+    const int item = __builtin_amdgcn_readfirstlane(s_item);
+    m = __builtin_amdgcn_readfirstlane(s_mol);
+    local = __builtin_amdgcn_readfirstlane(s_local);
+    __syncthreads();
+    return item < P.nitems;
+}
+
+// OFFQ: the tip has charge sites at a nonzero z offset (compiled out when it has none).
+template <int MODEL, bool HASQ0, int V, bool OFFQ>
+__global__ __launch_bounds__(256, 3) void k_batch_grid(const PpmMolDesc* __restrict__ mols, PpmBatchParams P,
+                                                       const float4* __restrict__ atoms, const float* __restrict__ cpar,
+                                                       float4* __restrict__ grids, Queue* q) {
+    __shared__ GridShared sh;
+    int m, local, done_m = -1;
+    while (take_item(mols, P, q, done_m, m, local)) {
+        done_m = -1;
+        if (local >= mols[m].n_grid_items) continue;
+        do_grid_item<MODEL, HASQ0, V, OFFQ>(mols[m], P, local, atoms, cpar, grids, sh);
+        done_m = m;
+    }
+}
+
+__global__ __launch_bounds__(256, 4) void k_batch_relax(const PpmMolDesc* __restrict__ mols, PpmBatchParams P,
+                                                        const float4* __restrict__ grids, float4* __restrict__ FEs,
+                                                        float4* __restrict__ PPs, float* __restrict__ df,
+                                                        const float* __restrict__ dfW, const int* __restrict__ dfStart,
+                                                        Queue* q) {
+    int m, local;
+    while (take_item(mols, P, q, -1, m, local)) {
         const PpmMolDesc& d = mols[m];
-        signal_m = -1;
-        if (local < d.n_grid_items) {
-            if constexpr (GRID) {
-                __shared__ GridShared sh;
-                do_grid_item<MODEL, HASQ0, V, OFFQ>(d, P, local, atoms, cpar, grids, sh);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-                __syncthreads();            // every thread's tile stores precede the signal
-                signal_m = m;
-            }
-        } else if (P.mode != PPM_BATCH_GRID_ONLY) {
-            if (threadIdx.x == 0) {
-                // relaxed polling (no cache invalidation per poll), one acquire after the wait
-                int spins = 0;
-                while (__hip_atomic_load(&done[m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < d.n_grid_items) {
-                    __builtin_amdgcn_s_sleep(8);
-                    if (++spins > kSpinLimit) {
-                        atomicOr(&q->error, 1);
-                        break;
-                    }
-                }
-            }
-            __syncthreads();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            do_relax_item(d, P, local - d.n_grid_items, grids, FEs, PPs, df, dfW, dfStart, &flags[m]);
-        }
+        if (local < d.n_grid_items) continue;
+        if (threadIdx.x == 0 && q_done(q)[m] < d.n_grid_items) atomicOr(&q->error, 1);
+        do_relax_item(d, P, local - d.n_grid_items, grids, FEs, PPs, df, dfW, dfStart, &q_flag(q, P.nmol)[m]);
     }
 }
 
 template <int MODEL, bool HASQ0, bool OFFQ>
 void launch_v(int V, dim3 grd, hipStream_t st, const PpmMolDesc* mols, const PpmBatchParams& P, const float4* atoms,
-              const float* cpar, float4* grids, float4* FEs, float4* PPs, float* df, const float* dfW,
-              const int* dfStart, Queue* q) {
+              const float* cpar, float4* grids, Queue* q) {
     if (V == 8)
-        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 8, OFFQ, true>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
-                           PPs, df, dfW, dfStart, q);
+        hipLaunchKernelGGL((k_batch_grid<MODEL, HASQ0, 8, OFFQ>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, q);
     else
-        hipLaunchKernelGGL((k_batch<MODEL, HASQ0, 4, OFFQ, true>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, FEs,
-                           PPs, df, dfW, dfStart, q);
+        hipLaunchKernelGGL((k_batch_grid<MODEL, HASQ0, 4, OFFQ>), grd, dim3(256), 0, st, mols, P, atoms, cpar, grids, q);
 }
 
 template <int MODEL>
-void launch_q(bool hasq0, bool offq, int V, dim3 grd, hipStream_t st, const PpmMolDesc* mols,
-              const PpmBatchParams& P, const float4* atoms, const float* cpar, float4* grids, float4* FEs,
-              float4* PPs, float* df, const float* dfW, const int* dfStart, Queue* q) {
+void launch_q(bool hasq0, bool offq, int V, dim3 grd, hipStream_t st, const PpmMolDesc* mols, const PpmBatchParams& P,
+              const float4* atoms, const float* cpar, float4* grids, Queue* q) {
     if (hasq0) {
-        if (offq) launch_v<MODEL, true, true>(V, grd, st, mols, P, atoms, cpar, grids, FEs, PPs, df, dfW, dfStart, q);
-        else launch_v<MODEL, true, false>(V, grd, st, mols, P, atoms, cpar, grids, FEs, PPs, df, dfW, dfStart, q);
+        if (offq) launch_v<MODEL, true, true>(V, grd, st, mols, P, atoms, cpar, grids, q);
+        else launch_v<MODEL, true, false>(V, grd, st, mols, P, atoms, cpar, grids, q);
     } else {
-        if (offq) launch_v<MODEL, false, true>(V, grd, st, mols, P, atoms, cpar, grids, FEs, PPs, df, dfW, dfStart, q);
-        else launch_v<MODEL, false, false>(V, grd, st, mols, P, atoms, cpar, grids, FEs, PPs, df, dfW, dfStart, q);
+        if (offq) launch_v<MODEL, false, true>(V, grd, st, mols, P, atoms, cpar, grids, q);
+        else launch_v<MODEL, false, false>(V, grd, st, mols, P, atoms, cpar, grids, q);
     }
 }
 
@@ -360,14 +344,20 @@ int launch_batch(const PpmMolDesc* mols, const PpmBatchParams& P, const float* a
     float4* gr = reinterpret_cast<float4*>(grids);
     float4* fe = reinterpret_cast<float4*>(FEs);
     float4* pp = reinterpret_cast<float4*>(PPs);
-    if (P.mode == PPM_BATCH_RELAX_ONLY)      // no pair law takes part
-        hipLaunchKernelGGL((k_batch<PPM_MODEL_LJ, false, 8, false, false>), grd, dim3(256), 0, stream, mols, P, at, cpar,
-                           gr, fe, pp, df, dfW, dfStart, q);
-    else if (P.model == PPM_MODEL_LJ)
-        launch_q<PPM_MODEL_LJ>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, fe, pp, df, dfW, dfStart, q);
-    else
-        launch_q<PPM_MODEL_MORSE>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, fe, pp, df, dfW, dfStart, q);
-    return check_launch("batch");
+    if (P.mode != PPM_BATCH_RELAX_ONLY) {
+        if (P.model == PPM_MODEL_LJ) launch_q<PPM_MODEL_LJ>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, q);
+        else launch_q<PPM_MODEL_MORSE>(hasq0, offq, P.vz, grd, stream, mols, P, at, cpar, gr, q);
+        if (int r = check_launch("batch_grid")) return r;
+    }
+    if (P.mode == PPM_BATCH_FUSED) {
+        hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, stream, q, P.nmol, 1);
+        if (int r = check_launch("batch_reset")) return r;
+    }
+    if (P.mode != PPM_BATCH_GRID_ONLY) {
+        hipLaunchKernelGGL(k_batch_relax, grd, dim3(256), 0, stream, mols, P, gr, fe, pp, df, dfW, dfStart, q);
+        if (int r = check_launch("batch_relax")) return r;
+    }
+    return PPM_OK;
 }
 
 int launch_batch_noalloc(const PpmMolDesc* mols, const PpmBatchParams& P, const float* atoms, const float* cpar,
