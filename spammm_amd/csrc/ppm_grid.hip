@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void k_grid_project(const float4* __restrict__
 
 // The interpolated form: workgroup (blockIdx.x, blockIdx.y) takes the (x,y) and z block (two levels: of
 // 32 voxels a side, one level: 16) of the planes [klo, kend); blocks are aligned to plane 0.
-template <int MODEL, bool HASQ0, bool OFFS, bool TWO, typename ACC>
+template <int MODEL, bool HASQ0, bool OFFS, bool TWO, typename ACC, bool BASE>
 __global__ __launch_bounds__(256, sizeof(ACC) == 8 ? 1 : TWO ? 2 : 3) void k_grid_far(
     const float4* __restrict__ atoms, const float* __restrict__ cpar, GridArgs a, float4* __restrict__ out,
     const float4* base, int klo, int kend, int split) {
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256, sizeof(ACC) == 8 ? 1 : TWO ? 2 : 3) void k_gri
     constexpr int B = TWO ? 2 * gf::kB : gf::kB;
     const int nbx = (a.nx + B - 1) / B;
     const int by = (int)blockIdx.x / nbx, bx = (int)blockIdx.x - by * nbx;
-    gf::far_blocks<MODEL, HASQ0, OFFS ? kOffDynamic : kOffNone, TWO, ACC>(
+    gf::far_blocks<MODEL, HASQ0, OFFS ? kOffDynamic : kOffNone, TWO, ACC, BASE>(
         s, atoms, cpar, a, bx * B, by * B, (klo / B + (int)blockIdx.y) * B, (int)blockIdx.z * (TWO ? 8 : 1) / split,
         ((int)blockIdx.z + 1) * (TWO ? 8 : 1) / split, klo, kend, out, base);
 }
@@ -746,10 +746,13 @@ int launch_far(const float4* atoms, const float* cpar, const GridArgs& a, float4
     const unsigned nxy = (unsigned)(((a.nx + B - 1) / B) * ((a.ny + B - 1) / B)), nz = (kend - 1) / B - klo / B + 1;
     const int split = TWO ? far_split(a, (double)nxy * nz) : 1;
     const dim3 grd(nxy, nz, (unsigned)split), blk(256);
-#define PPM_FAR(OF, AC) \
-    hipLaunchKernelGGL((k_grid_far<MODEL, HASQ0, OF, TWO, AC>), grd, blk, 0, st, atoms, cpar, a, out, base, klo, kend, split)
-    if (acc64) { if (a.noff) PPM_FAR(true, double); else PPM_FAR(false, double); }
-    else { if (a.noff) PPM_FAR(true, float); else PPM_FAR(false, float); }
+#define PPM_FAR(OF, AC, BA)                                                                                          \
+    hipLaunchKernelGGL((k_grid_far<MODEL, HASQ0, OF, TWO, AC, BA>), grd, blk, 0, st, atoms, cpar, a, out, base, klo, kend, \
+                       split)
+#define PPM_FAR_BASE(OF, AC) do { if (base) PPM_FAR(OF, AC, true); else PPM_FAR(OF, AC, false); } while (0)
+    if (acc64) { if (a.noff) PPM_FAR_BASE(true, double); else PPM_FAR_BASE(false, double); }
+    else { if (a.noff) PPM_FAR_BASE(true, float); else PPM_FAR_BASE(false, float); }
+#undef PPM_FAR_BASE
 #undef PPM_FAR
     return check_launch("grid_project_far");
 }

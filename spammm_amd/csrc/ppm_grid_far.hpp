@@ -33,6 +33,7 @@ constexpr int kM = 8;              // Chebyshev nodes per axis
 constexpr int kB = 16;             // voxels per axis of a block
 constexpr int kList = 512;         // sites near a workgroup's blocks that LDS holds at a time
 constexpr float kRatio = 10.0f;       // near: closer than kRatio half-widths
+constexpr int kBase = 8;           // planes of a base grid read at a time
 constexpr int kMinMid = 6;         // fewer sites than this are cheaper summed at the voxels
 
 // cos((2 i + 1) pi / 16): the nodes on [-1, 1], descending
@@ -417,8 +418,9 @@ __device__ __forceinline__ int collect(Shared& s, const float4* __restrict__ ato
 // The 16^3 blocks of one workgroup of 256 threads: TWO: the 2^3 blocks whose first voxel is (i0, j0, k0),
 // otherwise the one block there.  Voxels with klo <= ic < kend are stored at out[(ic - klo) * ncol + col];
 // base as for grid_tile.  Every thread of the workgroup must call it.
-// ACC: float, or double (pair terms at the nodes and all sums in FP64, terms at the voxels in FP32).
-template <int MODEL, bool HASQ0, int OFF, bool TWO, typename ACC>
+// ACC: float, or double (pair terms at the nodes and all sums in FP64, terms at the voxels in FP32).  BASE: base is added
+// (a form of its own: its loads cost the others 1 to 3 %).
+template <int MODEL, bool HASQ0, int OFF, bool TWO, typename ACC, bool BASE = false>
 __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__ atoms, const float* __restrict__ cpar,
                                            const GridArgs& a, int i0, int j0, int k0, int sub0, int sub1, int klo,
                                            int kend, float4* __restrict__ out, const float4* base) {
@@ -569,20 +571,31 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         }
         if (bi + x < a.nx && bj + y < a.ny) {
             const int col = (bj + y) * a.nx + bi + x;
+            // base may be out: the compiler keeps a load behind the stores before it, so eight planes of base are
+            // read before the first of them is stored (480x480x149 with a base: 629 -> 522 us)
 #pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                const int ic = bk + k;
-                if (ic < klo || ic >= kend) continue;
-                float4 v = make_float4((float)f[k][0], (float)f[k][1], (float)f[k][2], (float)f[k][3]);
-                if (base) {
-                    const float4 b = base[(size_t)(ic - klo) * a.ncol + col];
-                    v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
+            for (int k0 = 0; k0 < kB; k0 += kBase) {
+                float4 b[kBase];
+                if constexpr (BASE) {
+#pragma unroll
+                    for (int k = 0; k < kBase; ++k) {
+                        const int ic = min(max(bk + k0 + k, klo), kend - 1);
+                        b[k] = base[(size_t)(ic - klo) * a.ncol + col];
+                    }
                 }
-                if (a.cap) {
-                    const float renorm = 100.0f / fabsf(v.w);
-                    if (renorm < 1.0f) { v.x *= renorm; v.y *= renorm; v.z *= renorm; v.w *= renorm; }
+#pragma unroll
+                for (int k = 0; k < kBase; ++k) {
+                    const int ic = bk + k0 + k;
+                    if (ic < klo || ic >= kend) continue;
+                    float4 v = make_float4((float)f[k0 + k][0], (float)f[k0 + k][1], (float)f[k0 + k][2],
+                                           (float)f[k0 + k][3]);
+                    if constexpr (BASE) { v.x += b[k].x; v.y += b[k].y; v.z += b[k].z; v.w += b[k].w; }
+                    if (a.cap) {
+                        const float renorm = 100.0f / fabsf(v.w);
+                        if (renorm < 1.0f) { v.x *= renorm; v.y *= renorm; v.z *= renorm; v.w *= renorm; }
+                    }
+                    out[(size_t)(ic - klo) * a.ncol + col] = v;
                 }
-                out[(size_t)(ic - klo) * a.ncol + col] = v;
             }
         }
         __syncthreads();                            // the next block reuses the lists and buffers
