@@ -164,13 +164,14 @@ int ppm_grid_project(int model, const float* atoms, const float* cpar, int na,
                      int npbc_a, int npbc_b, const float lvA[3], const float lvB[3],
                      int cap, float* grid, void* stream);
 
-/* ppm_grid_project with each voxel's pair terms, evaluated in FP32 exactly as there, summed in
- * FP64 and rounded once to the FP32 output.  Same arguments, pair laws, images and rescale
+/* ppm_grid_project as a direct sum: every pair term evaluated in FP32 at the voxel, summed in
+ * FP64 and rounded once to the FP32 output, at any grid size.  Same arguments, pair laws, images and rescale
  * (evalLJC_QZs_toImg / evalMorseC_QZs_toImg, kernels/AFM.cl:916-1056, whose FP32 sum it
  * refines).  Above a neutral molecule the thousands of terms of a voxel cancel to ~1e-2 of
  * their magnitude and the FP32 running sum dominates the field's error; this form removes that
- * part (3-6x lower error there) at ~1.55x the time (8 voxels per thread), for uses bound by
- * the field's own accuracy. */
+ * part (3-6x lower error there) at ~1.55x the time of the FP32 direct sum (8 voxels per thread),
+ * for uses bound by the field's own accuracy.  ppm_grid_project itself sums the far atoms of
+ * larger grids at the nodes of voxel blocks, which this form does not. */
 int ppm_grid_project_acc64(int model, const float* atoms, const float* cpar, int na,
                            const PpmGridSpec* spec, const float Qs[4], const float QZs[4],
                            int npbc_a, int npbc_b, const float lvA[3], const float lvB[3],

@@ -149,11 +149,11 @@ __device__ void do_grid_item(const PpmMolDesc& d, const PpmBatchParams& P, int l
             gc::grid_tile<MODEL, HASQ0, V, true, OFF>(at, cp, a, sh.sites, x * 256 + threadIdx.x, d.klo + z * V, kend,
                                                       out, d.klo);
         else if (MODEL == PPM_MODEL_LJ && n.level == 2)
-            gf::far_blocks<MODEL, HASQ0, OFF, true, float>(sh.far, at, cp, a, x * 32, y * 32, (d.klo / 32 + z) * 32,
+            gf::far_blocks<MODEL, HASQ0, OFF, true>(sh.far, at, cp, a, x * 32, y * 32, (d.klo / 32 + z) * 32,
                                                            part * 8 / n.split, (part + 1) * 8 / n.split, d.klo, kend,
                                                            out, nullptr);
         else
-            gf::far_blocks<MODEL, HASQ0, OFF, false, float>(sh.far, at, cp, a, x * 16, y * 16, (d.klo / 16 + z) * 16, 0,
+            gf::far_blocks<MODEL, HASQ0, OFF, false>(sh.far, at, cp, a, x * 16, y * 16, (d.klo / 16 + z) * 16, 0,
                                                             1, d.klo, kend, out, nullptr);
     }
 }

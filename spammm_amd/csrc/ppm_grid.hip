@@ -48,15 +48,15 @@ __global__ __launch_bounds__(256) void k_grid_project(const float4* __restrict__
 
 // The interpolated form: workgroup (blockIdx.x, blockIdx.y) takes the (x,y) and z block (two levels: of
 // 32 voxels a side, one level: 16) of the planes [klo, kend); blocks are aligned to plane 0.
-template <int MODEL, bool HASQ0, bool OFFS, bool TWO, typename ACC, bool BASE>
-__global__ __launch_bounds__(256, sizeof(ACC) == 8 ? 1 : TWO ? 2 : 3) void k_grid_far(
+template <int MODEL, bool HASQ0, bool OFFS, bool TWO, bool BASE>
+__global__ __launch_bounds__(256, TWO ? 2 : 3) void k_grid_far(
     const float4* __restrict__ atoms, const float* __restrict__ cpar, GridArgs a, float4* __restrict__ out,
     const float4* base, int klo, int kend, int split) {
     __shared__ gf::Shared s;
     constexpr int B = TWO ? 2 * gf::kB : gf::kB;
     const int nbx = (a.nx + B - 1) / B;
     const int by = (int)blockIdx.x / nbx, bx = (int)blockIdx.x - by * nbx;
-    gf::far_blocks<MODEL, HASQ0, OFFS ? kOffDynamic : kOffNone, TWO, ACC, BASE>(
+    gf::far_blocks<MODEL, HASQ0, OFFS ? kOffDynamic : kOffNone, TWO, BASE>(
         s, atoms, cpar, a, bx * B, by * B, (klo / B + (int)blockIdx.y) * B, (int)blockIdx.z * (TWO ? 8 : 1) / split,
         ((int)blockIdx.z + 1) * (TWO ? 8 : 1) / split, klo, kend, out, base);
 }
@@ -740,19 +740,16 @@ int far_split(const GridArgs& a, double nb) {
 }
 
 template <int MODEL, bool HASQ0, bool TWO>
-int launch_far(const float4* atoms, const float* cpar, const GridArgs& a, float4* out, const float4* base, bool acc64,
-               hipStream_t st, int klo, int kend) {
+int launch_far(const float4* atoms, const float* cpar, const GridArgs& a, float4* out, const float4* base, hipStream_t st,
+               int klo, int kend) {
     constexpr int B = TWO ? 2 * gf::kB : gf::kB;
     const unsigned nxy = (unsigned)(((a.nx + B - 1) / B) * ((a.ny + B - 1) / B)), nz = (kend - 1) / B - klo / B + 1;
     const int split = TWO ? far_split(a, (double)nxy * nz) : 1;
     const dim3 grd(nxy, nz, (unsigned)split), blk(256);
-#define PPM_FAR(OF, AC, BA)                                                                                          \
-    hipLaunchKernelGGL((k_grid_far<MODEL, HASQ0, OF, TWO, AC, BA>), grd, blk, 0, st, atoms, cpar, a, out, base, klo, kend, \
-                       split)
-#define PPM_FAR_BASE(OF, AC) do { if (base) PPM_FAR(OF, AC, true); else PPM_FAR(OF, AC, false); } while (0)
-    if (acc64) { if (a.noff) PPM_FAR_BASE(true, double); else PPM_FAR_BASE(false, double); }
-    else { if (a.noff) PPM_FAR_BASE(true, float); else PPM_FAR_BASE(false, float); }
-#undef PPM_FAR_BASE
+#define PPM_FAR(OF, BA) \
+    hipLaunchKernelGGL((k_grid_far<MODEL, HASQ0, OF, TWO, BA>), grd, blk, 0, st, atoms, cpar, a, out, base, klo, kend, split)
+    if (a.noff) { if (base) PPM_FAR(true, true); else PPM_FAR(true, false); }
+    else { if (base) PPM_FAR(false, true); else PPM_FAR(false, false); }
 #undef PPM_FAR
     return check_launch("grid_project_far");
 }
@@ -763,10 +760,11 @@ int dispatch(const float4* atoms, const float* cpar, const GridArgs& a, float4* 
     const bool dcz = (a.dC[0] == 0.f && a.dC[1] == 0.f);
     const int kend = klo + nzw;
     dim3 blk(256);
-    const int level = far_level(a, MODEL);
+    // FP64 sums of the FP32 terms at every voxel: the direct sum at any size
+    const int level = acc64 ? 0 : far_level(a, MODEL);
     if constexpr (MODEL == PPM_MODEL_LJ)
-        if (level == 2) return launch_far<MODEL, HASQ0, true>(atoms, cpar, a, out, base, acc64, st, klo, kend);
-    if (level) return launch_far<MODEL, HASQ0, false>(atoms, cpar, a, out, base, acc64, st, klo, kend);
+        if (level == 2) return launch_far<MODEL, HASQ0, true>(atoms, cpar, a, out, base, st, klo, kend);
+    if (level) return launch_far<MODEL, HASQ0, false>(atoms, cpar, a, out, base, st, klo, kend);
     if (acc64) {          // FP64 sums: 8 voxels per thread (16 would need 128 VGPRs of sums alone)
         const int V = dcz ? 8 : 4;
         dim3 grd((a.ncol + 255) / 256, (nzw + V - 1) / V);

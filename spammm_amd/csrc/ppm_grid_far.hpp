@@ -170,66 +170,59 @@ __device__ __forceinline__ bool is_near(const Site& S, const Centre& c, float r2
     return !(dx * dx + dy * dy + dz * dz >= r2);
 }
 
-__device__ __forceinline__ double inv_sqrt(double x) { return 1.0 / sqrt(x); }
-__device__ __forceinline__ float inv_sqrt(float x) { return gc::rsq(x); }
-__device__ __forceinline__ double exp_2(double x) { return exp2(x); }
-__device__ __forceinline__ float exp_2(float x) { return gc::ex2(x); }
-__device__ __forceinline__ float mad(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ __forceinline__ double mad(double a, double b, double c) { return fma(a, b, c); }
-
 // One site at N points of a column (same dx, dy; dz[k] = oz[k] - sz): f[k] += (Fx, Fy, Fz, E).
-// The pair laws are grid_tile's.  T: type of the terms, ACC: of the sums.
-template <int MODEL, bool HASQ0, int OFF, int N, typename T, typename ACC>
-__device__ __forceinline__ void add_site(const Site& S, const GridArgs& a, T dx, T dy, T sz, const float (&oz)[N],
-                                         ACC (&f)[N][4]) {
-    const T dxy2 = mad(dx, dx, mad(dy, dy, (T)kR2SAFE));
-    const T qq0 = (T)S.q * (T)a.q0;
+// The pair laws are grid_tile's.
+template <int MODEL, bool HASQ0, int OFF, int N>
+__device__ __forceinline__ void add_site(const Site& S, const GridArgs& a, float dx, float dy, float sz,
+                                         const float (&oz)[N], float (&f)[N][4]) {
+    const float dxy2 = fmaf(dx, dx, fmaf(dy, dy, kR2SAFE));
+    const float qq0 = S.q * a.q0;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        const T dz = (T)oz[k] - sz;
-        const T r2 = mad(dz, dz, dxy2);
-        const T ir = inv_sqrt(r2);
-        const T ir2 = ir * ir;
-        T fr;
+        const float dz = oz[k] - sz;
+        const float r2 = fmaf(dz, dz, dxy2);
+        const float ir = gc::rsq(r2);
+        const float ir2 = ir * ir;
+        float fr;
         if (MODEL == PPM_MODEL_LJ) {
-            const T ir6 = ir2 * ir2 * ir2;
-            const T t6 = mad((T)S.c1, ir6, -(T)S.c0), t7 = mad((T)S.c3, ir6, -(T)S.c2);
+            const float ir6 = ir2 * ir2 * ir2;
+            const float t6 = fmaf(S.c1, ir6, -S.c0), t7 = fmaf(S.c3, ir6, -S.c2);
             if (HASQ0) {
-                const T ec = qq0 * ir;
-                f[k][3] = mad((ACC)t6, (ACC)ir6, f[k][3] + (ACC)ec);
-                fr = mad(t7, ir6, ec) * ir2;
+                const float ec = qq0 * ir;
+                f[k][3] = fmaf(t6, ir6, f[k][3] + ec);
+                fr = fmaf(t7, ir6, ec) * ir2;
             } else {
-                f[k][3] = mad((ACC)t6, (ACC)ir6, f[k][3]);
+                f[k][3] = fmaf(t6, ir6, f[k][3]);
                 fr = t7 * ir6 * ir2;
             }
         } else {
-            const T r = r2 * ir;
-            const T ex = exp_2(mad((T)S.c2, r, (T)S.c0));
-            const T Ae = (T)S.c1 * ex;
-            f[k][3] = mad((ACC)(ex - (T)2), (ACC)Ae, f[k][3]);
-            fr = (T)S.c3 * (Ae * (ex - (T)1)) * ir;
+            const float r = r2 * ir;
+            const float ex = gc::ex2(fmaf(S.c2, r, S.c0));
+            const float Ae = S.c1 * ex;
+            f[k][3] = fmaf(ex - 2.0f, Ae, f[k][3]);
+            fr = S.c3 * (Ae * (ex - 1.0f)) * ir;
             if (HASQ0) {
-                const T ec = qq0 * ir;
-                fr = mad(ec, ir2, fr);
-                f[k][3] += (ACC)ec;
+                const float ec = qq0 * ir;
+                fr = fmaf(ec, ir2, fr);
+                f[k][3] += ec;
             }
         }
-        f[k][0] = mad((ACC)fr, (ACC)dx, f[k][0]);
-        f[k][1] = mad((ACC)fr, (ACC)dy, f[k][1]);
-        f[k][2] = mad((ACC)fr, (ACC)dz, f[k][2]);
+        f[k][0] = fmaf(fr, dx, f[k][0]);
+        f[k][1] = fmaf(fr, dy, f[k][1]);
+        f[k][2] = fmaf(fr, dz, f[k][2]);
     }
     auto charge = [&](float qf, float zf) {
-        const T qo = (T)S.q * (T)qf, zo = (T)zf;
+        const float qo = S.q * qf, zo = zf;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const T dzo = ((T)oz[k] - sz) + zo;
-            const T iro = inv_sqrt(mad(dzo, dzo, dxy2));
-            const T eo = qo * iro;
-            const T fro = eo * iro * iro;
-            f[k][0] = mad((ACC)fro, (ACC)dx, f[k][0]);
-            f[k][1] = mad((ACC)fro, (ACC)dy, f[k][1]);
-            f[k][2] = mad((ACC)fro, (ACC)dzo, f[k][2]);
-            f[k][3] += (ACC)eo;
+            const float dzo = (oz[k] - sz) + zo;
+            const float iro = gc::rsq(fmaf(dzo, dzo, dxy2));
+            const float eo = qo * iro;
+            const float fro = eo * iro * iro;
+            f[k][0] = fmaf(fro, dx, f[k][0]);
+            f[k][1] = fmaf(fro, dy, f[k][1]);
+            f[k][2] = fmaf(fro, dzo, f[k][2]);
+            f[k][3] += eo;
         }
     };
     if constexpr (OFF == gc::kOffStatic) {
@@ -263,8 +256,7 @@ __device__ __forceinline__ void ranks(bool f, bool g, int (&cnt)[2][4], int& rf,
 }
 
 // Sum over the 4 waves of the node sums f (lane = column y * 8 + x, k = z) into dst[channel][z * 64 + lane].
-template <typename ACC>
-__device__ __forceinline__ void reduce_nodes(Shared& s, const ACC (&f)[kM][4], float (*dst)[kM * kM * kM]) {
+__device__ __forceinline__ void reduce_nodes(Shared& s, const float (&f)[kM][4], float (*dst)[kM * kM * kM]) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     float* part = &s.b[0][0];                       // 2 x 2048 floats, and the third part in a
     float* buf[3] = {part, part + 2048, &s.a[0][0]};
@@ -272,7 +264,7 @@ __device__ __forceinline__ void reduce_nodes(Shared& s, const ACC (&f)[kM][4], f
 #pragma unroll
         for (int k = 0; k < kM; ++k)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) buf[w - 1][(c * kM + k) * 64 + lane] = (float)f[k][c];
+            for (int c = 0; c < 4; ++c) buf[w - 1][(c * kM + k) * 64 + lane] = f[k][c];
     __syncthreads();
     float v[kM][4];
     if (w == 0)
@@ -281,7 +273,7 @@ __device__ __forceinline__ void reduce_nodes(Shared& s, const ACC (&f)[kM][4], f
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int i = (c * kM + k) * 64 + lane;
-                v[k][c] = ((float)f[k][c] + buf[0][i]) + (buf[1][i] + buf[2][i]);
+                v[k][c] = (f[k][c] + buf[0][i]) + (buf[1][i] + buf[2][i]);
             }
     if (dst == nullptr) {                           // into a, which buf[2] is part of: one wave, in order
         if (w == 0)
@@ -339,8 +331,7 @@ __device__ __forceinline__ void add_top(Shared& s, int hx, int hy, int hz) {
 
 // f = the polynomial through the node values a at this thread's column (x, y) = (tid & 15, tid >> 4)
 // of the block's voxels: z in registers, then y and x through LDS, 8 planes at a time.
-template <typename ACC>
-__device__ __forceinline__ void interpolate(Shared& s, ACC (&f)[kB][4]) {
+__device__ __forceinline__ void interpolate(Shared& s, float (&f)[kB][4]) {
     const int lane = threadIdx.x & 63, ch = threadIdx.x >> 6;
     const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
     float wx[kM], v[kM], z[kB];
@@ -381,7 +372,7 @@ __device__ __forceinline__ void interpolate(Shared& s, ACC (&f)[kB][4]) {
                 float o = wx[0] * p0.x;
                 o = fmaf(wx[1], p0.y, o); o = fmaf(wx[2], p0.z, o); o = fmaf(wx[3], p0.w, o);
                 o = fmaf(wx[4], p1.x, o); o = fmaf(wx[5], p1.y, o); o = fmaf(wx[6], p1.z, o);
-                f[half * 8 + i][c] = (ACC)fmaf(wx[7], p1.w, o);
+                f[half * 8 + i][c] = fmaf(wx[7], p1.w, o);
             }
         }
     }
@@ -418,9 +409,8 @@ __device__ __forceinline__ int collect(Shared& s, const float4* __restrict__ ato
 // The 16^3 blocks of one workgroup of 256 threads: TWO: the 2^3 blocks whose first voxel is (i0, j0, k0),
 // otherwise the one block there.  Voxels with klo <= ic < kend are stored at out[(ic - klo) * ncol + col];
 // base as for grid_tile.  Every thread of the workgroup must call it.
-// ACC: float, or double (pair terms at the nodes and all sums in FP64, terms at the voxels in FP32).  BASE: base is added
-// (a form of its own: its loads cost the others 1 to 3 %).
-template <int MODEL, bool HASQ0, int OFF, bool TWO, typename ACC, bool BASE = false>
+// BASE: base is added (a form of its own: its loads cost the others 1 to 3 %).
+template <int MODEL, bool HASQ0, int OFF, bool TWO, bool BASE = false>
 __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__ atoms, const float* __restrict__ cpar,
                                            const GridArgs& a, int i0, int j0, int k0, int sub0, int sub1, int klo,
                                            int kend, float4* __restrict__ out, const float4* base) {
@@ -453,7 +443,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         const Centre c = centre_of(a, i0, j0, k0, kB - 0.5);
         float ox, oy, oz[kM];
         node_offsets(c, kB - 0.5f, ox, oy, oz);
-        ACC f[kM][4];
+        float f[kM][4];
 #pragma unroll
         for (int k = 0; k < kM; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
         int nfar = 0;
@@ -465,9 +455,8 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                                    for (int j = wave; j < n; j += 4) {
                                        const Site S = Sn;
                                        Sn = s.tile[min(j + 4, n - 1)];
-                                       add_site<MODEL, HASQ0, OFF, kM, ACC, ACC>(
-                                           S, a, (ACC)ox - ((ACC)S.x - (ACC)c.x), (ACC)oy - ((ACC)S.y - (ACC)c.y),
-                                           (ACC)S.z - (ACC)c.z, oz, f);
+                                       add_site<MODEL, HASQ0, OFF, kM>(S, a, ox - (S.x - c.x), oy - (S.y - c.y),
+                                                                       S.z - c.z, oz, f);
                                    }
                                });
         top = nfar > 0;
@@ -513,7 +502,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         {
             float ox, oy, oz[kM];
             node_offsets(c, 0.5f * (kB - 1), ox, oy, oz);
-            ACC f[kM][4];
+            float f[kM][4];
 #pragma unroll
             for (int k = 0; k < kM; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
             for (int r = 0; r < rounds; ++r) {
@@ -526,15 +515,13 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                 for (int j = wave; j < nmid; j += 4) {
                     const Site S = Sn;
                     Sn = s.list[s.mid[min(j + 4, nmid - 1)]];
-                    add_site<MODEL, HASQ0, OFF, kM, ACC, ACC>(S, a, (ACC)ox - ((ACC)S.x - (ACC)c.x),
-                                                             (ACC)oy - ((ACC)S.y - (ACC)c.y),
-                                                             (ACC)S.z - (ACC)c.z, oz, f);
+                    add_site<MODEL, HASQ0, OFF, kM>(S, a, ox - (S.x - c.x), oy - (S.y - c.y), S.z - c.z, oz, f);
                 }
             }
-            if (top || mids > 0) reduce_nodes<ACC>(s, f, nullptr);
+            if (top || mids > 0) reduce_nodes(s, f, nullptr);
         }
         const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-        ACC f[kB][4];
+        float f[kB][4];
         if (top || mids > 0) {
             if (top) add_top(s, hx, hy, hz);
             interpolate(s, f);
@@ -555,7 +542,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                 split(n, nmid, nnear);
             }
             auto site = [&](const Site& S) {
-                add_site<MODEL, HASQ0, OFF, kB, float, ACC>(S, a, px - S.x, py - S.y, S.z, pz, f);
+                add_site<MODEL, HASQ0, OFF, kB>(S, a, px - S.x, py - S.y, S.z, pz, f);
             };
             auto all = [&](const unsigned short* idx, int n) {
                 if (n == 0) return;
@@ -587,8 +574,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                 for (int k = 0; k < kBase; ++k) {
                     const int ic = bk + k0 + k;
                     if (ic < klo || ic >= kend) continue;
-                    float4 v = make_float4((float)f[k0 + k][0], (float)f[k0 + k][1], (float)f[k0 + k][2],
-                                           (float)f[k0 + k][3]);
+                    float4 v = make_float4(f[k0 + k][0], f[k0 + k][1], f[k0 + k][2], f[k0 + k][3]);
                     if constexpr (BASE) { v.x += b[k].x; v.y += b[k].y; v.z += b[k].z; v.w += b[k].w; }
                     if (a.cap) {
                         const float renorm = 100.0f / fabsf(v.w);
