@@ -402,7 +402,7 @@ constexpr int kNearList = 512;
 // than the field: at 10, gradients on a 0.05 A grid were up to 5 times further off FP64 than the direct form's.
 constexpr double kAdjRatio = 12.5;
 inline double adj_near2(const GridArgs& a) {
-    return gf::near2(a, false) * (kAdjRatio / gf::kRatio) * (kAdjRatio / gf::kRatio);
+    return gf::half2(a, false) * kAdjRatio * kAdjRatio;
 }
 
 struct AdjFar {
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(256, 3) void k_adj_far(const float4* __restrict__ a
             site(ok ? i : s_end - 1, at, p0, p1, K);
             gc::Site S{};
             S.x = at.x; S.y = at.y; S.z = at.z;
-            const bool nr = ok && gf::is_near(S, c, near_r2, zlo, zhi);
+            const bool nr = ok && gf::closer(S, c, near_r2, zlo, zhi);
             int rk, nk, ro, no;
             gf::ranks(nr, ok && !nr, s.cnt, rk, nk, ro, no);
             if (nr) s.list[n_near + rk] = i;
@@ -728,7 +728,8 @@ bool lj_16_voxels(int ncol, int nzw) {
 // 3.5e6 ms: the card's rate and one workgroup's serial time.  300x300x62 planes, 1800 sites: s = 1, 2,
 // 4, 8 take 597, 459, 522, 714 us; 300x300x240: 722, 916, 1324, 2247.
 int far_split(const GridArgs& a, double nb) {
-    const double n = a.nsites, near = expected_near(a, near2(a, false)), mid = expected_near(a, near2(a, true));
+    const double n = a.nsites, near = expected_near(a, near2(a, PPM_MODEL_LJ, false)),
+                 mid = expected_near(a, near2(a, PPM_MODEL_LJ, true));
     const double F = 512.0 * (n - mid), S = 8.0 * (512.0 * (mid - near) + 4096.0 * near + 62e3);
     int best = 1;
     double t = 0.0;

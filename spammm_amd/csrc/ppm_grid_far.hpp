@@ -12,8 +12,10 @@
 //     8^3 nodes of the 32^3 voxels (512 instead of 32768), and that polynomial is evaluated at the
 //     nodes of each block.
 // No site is left out: every site enters every voxel once, through exactly one of the three sums.
-// The interpolation error of a site at distance d from the centre of a block of half-width h falls
-// as (d/h + sqrt((d/h)^2 - 1))^-8; kRatio h is where it passes below the FP32 rounding of the sums.
+// The interpolation error of a force r^-p at distance d from the centre of a block of half-width h is about
+// C(p + 7, 8) / 2^7 (h/d)^8 of it: the steeper the law, the larger (p = 2: 7e-10 at d = 10 h, 7: 2.3e-7, 13: 1e-5).
+// A site is near closer than kRatio h, and farther out while that error of its terms is above the FP32 rounding of
+// their sum (is_near).
 // Blocks are aligned to voxel 0 of the grid, whatever planes are stored, and which sums a site takes
 // depends on the block alone, so a z window has the bits of the same planes of the whole grid.
 //
@@ -32,7 +34,11 @@ using gc::Site;
 constexpr int kM = 8;              // Chebyshev nodes per axis
 constexpr int kB = 16;             // voxels per axis of a block
 constexpr int kList = 512;         // sites near a workgroup's blocks that LDS holds at a time
-constexpr float kRatio = 10.0f;       // near: closer than kRatio half-widths
+constexpr float kRatio = 10.0f;    // near: closer than kRatio half-widths
+constexpr float kTol = 0x1p-22f;   // and while the interpolation error is above this share of a site's terms
+// C(p + 7, 8) / 2^7 of the forces r^-7 and r^-13 (measured against FP64 over a block's voxels at 10 to 16 half-widths:
+// rms 0.8 to 1.1 of this, largest 1.4 to 3.1)
+constexpr float kErr6 = 23.5f, kErr12 = 984.f;
 constexpr int kBase = 8;           // planes of a base grid read at a time
 constexpr int kMinMid = 6;         // fewer sites than this are cheaper summed at the voxels
 
@@ -98,10 +104,23 @@ __host__ __device__ inline double step2(const GridArgs& a) {
     return m;
 }
 
-// Squared near radii: kRatio half-widths of a block, and of 2^3 blocks.
-__host__ __device__ inline double near2(const GridArgs& a, bool top) {
-    const double h = (top ? kB - 0.5 : 0.5 * (kB - 1)) * (double)kRatio;
+// Squared half-width of a block, and of 2^3 blocks.
+__host__ __device__ inline double half2(const GridArgs& a, bool top) {
+    const double h = top ? kB - 0.5 : 0.5 * (kB - 1);
     return step2(a) * (h * h);
+}
+
+// Squared near radius for the costs: at least kRatio half-widths, and for LJ what is_near gives an uncharged atom with
+// its minimum at 3.5 A (10.5 half-widths at 0.1 A, 13 at 0.05 A, 15 at 0.03 A).
+__host__ __device__ inline double near2(const GridArgs& a, int model, bool top) {
+    const double h2 = half2(a, top);
+    double q2 = (double)kRatio * (double)kRatio;
+    if (model == PPM_MODEL_LJ)
+        for (int i = 0; i < 40; ++i, q2 *= 1.03) {
+            const double d2 = q2 * h2, i2 = 12.25 / d2, t12 = 2.0 * i2 * i2 * i2, w = 1.0 / (q2 * q2 * q2 * q2);
+            if (w * ((double)kErr6 + (double)kErr12 * t12) <= (double)kTol * (1.0 + t12)) break;
+        }
+    return q2 * h2;
 }
 
 // Expected number of sites within r of a point of the molecule's plane, from the sites' area density
@@ -131,13 +150,13 @@ __host__ __device__ inline double expected_near(const GridArgs& a, double r2) {
 __host__ __device__ inline int far_level(const GridArgs& a, int model) {
     if (a.dC[0] != 0.f || a.dC[1] != 0.f) return 0;
     const double n = (double)a.nsites, vox = (double)a.nx * a.ny * a.nz;
-    const double near = expected_near(a, near2(a, false));
+    const double near = expected_near(a, near2(a, model, false));
     const double per = 512.0 * (n - near) + 4096.0 * near;
     auto blocks = [&](int b) { return (double)((a.nx + b - 1) / b) * ((a.ny + b - 1) / b) * ((a.nz + b - 1) / b); };
     double one = blocks(kB) * (per + 25e3);
     if (one < 362.0 * per) one = 362.0 * per;
     if (!(one + 5.8e7 < 0.85 * (vox * n + 5.8e7))) return 0;
-    const double nb = blocks(2 * kB), far = (n - expected_near(a, near2(a, true))) * nb;
+    const double nb = blocks(2 * kB), far = (n - expected_near(a, near2(a, model, true))) * nb;
     return model == PPM_MODEL_LJ && far >= (nb >= 150.0 ? 1e5 : 4e5) ? 2 : 1;
 }
 
@@ -161,13 +180,50 @@ __device__ __forceinline__ Centre centre_of(const GridArgs& a, int i0, int j0, i
     return c;
 }
 
-// Closer than r to the centre c, with every charge of the tip's sites (the tip charge at z offset
-// zo sees the site at S.z - zo; [zlo, zhi] spans 0 and the offsets).  A NaN position is near.
-__device__ __forceinline__ bool is_near(const Site& S, const Centre& c, float r2, float zlo, float zhi) {
+// What decides whether a site is near a block: the squared half-width, the span [zlo, zhi] of 0 and the tip charges'
+// z offsets, and the sum of the |charges|.
+struct NearRule {
+    float h2, zlo, zhi, q;
+};
+
+template <int OFF>
+__device__ __forceinline__ NearRule near_rule(const GridArgs& a, bool top) {
+    NearRule n{uniform((float)half2(a, top)), 0.f, 0.f, fabsf(a.q0)};
+#pragma unroll
+    for (int o = 0; o < 4; ++o)
+        if (OFF != gc::kOffNone && o < a.noff) {
+            n.zlo = fminf(n.zlo, a.zoff[o]);
+            n.zhi = fmaxf(n.zhi, a.zoff[o]);
+            n.q += fabsf(a.qoff[o]);
+        }
+    return n;
+}
+
+// Closer than r to the centre c, with every charge of the tip's sites (the tip charge at z offset zo sees the site at
+// S.z - zo; [zlo, zhi] spans 0 and the offsets).  A NaN position is.
+__device__ __forceinline__ bool closer(const Site& S, const Centre& c, float r2, float zlo, float zhi) {
     const float dx = S.x - c.x, dy = S.y - c.y;
     const float up = S.z - zlo - c.z, lo = S.z - zhi - c.z;      // the interval the charges span
     const float dz = lo > 0.f ? lo : (up < 0.f ? up : 0.f);
     return !(dx * dx + dy * dy + dz * dz >= r2);
+}
+
+// Near the centre c: closer than kRatio half-widths, or with an interpolation error above kTol of the site's terms.
+// LJ without charges, rms error against FP64 of the direct sum | with kRatio alone | so, relative, where kRatio alone is
+// worst: 0.04 A voxels at 3 A 9.5e-7 | 4.5e-6 | 2.7e-7, 0.03 A at 2 A 1.1e-6 | 2.5e-6 | 6.4e-7.
+template <int MODEL>
+__device__ __forceinline__ bool is_near(const Site& S, const Centre& c, const NearRule& n) {
+    if (closer(S, c, kRatio * kRatio * n.h2, n.zlo, n.zhi)) return true;
+    if constexpr (MODEL == PPM_MODEL_LJ) {
+        const float dx = S.x - c.x, dy = S.y - c.y, dz = S.z - c.z, dxy2 = dx * dx + dy * dy;
+        const float up = dz - n.zlo, lo = dz - n.zhi;
+        const float d2 = dxy2 + dz * dz, i2 = 1.0f / d2, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2;
+        const float fq = fmaxf(fabsf(up), fabsf(lo));            // the farthest charge
+        const float t6 = fabsf(S.c2) * i6, t12 = fabsf(S.c3) * i6 * i6;              // forces times distance
+        const float tc = fabsf(S.q) * n.q * sqrtf(d2) / (dxy2 + fq * fq);
+        return !(e4 * e4 * (kErr6 * t6 + kErr12 * t12) <= kTol * (t6 + t12 + tc));
+    }
+    return false;
 }
 
 // One site at N points of a column (same dx, dy; dz[k] = oz[k] - sz): f[k] += (Fx, Fy, Fz, E).
@@ -415,11 +471,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                                            const GridArgs& a, int i0, int j0, int k0, int sub0, int sub1, int klo,
                                            int kend, float4* __restrict__ out, const float4* base) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float zlo = 0.f, zhi = 0.f;                     // span of the tip charges' z offsets
-#pragma unroll
-    for (int o = 0; o < 4; ++o)
-        if (OFF != gc::kOffNone && o < a.noff) { zlo = fminf(zlo, a.zoff[o]); zhi = fmaxf(zhi, a.zoff[o]); }
-    const float r0 = uniform((float)near2(a, false)), r1 = uniform((float)near2(a, true));      // squared
+    const NearRule n0 = near_rule<OFF>(a, false), n1 = near_rule<OFF>(a, true);
 
     // offsets of this lane's column of nodes from a centre, for half-width `half` (voxels)
     auto node_offsets = [&](const Centre& c, float half, float& ox, float& oy, float (&oz)[kM]) {
@@ -447,7 +499,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
 #pragma unroll
         for (int k = 0; k < kM; ++k) f[k][0] = f[k][1] = f[k][2] = f[k][3] = 0;
         int nfar = 0;
-        total = collect<MODEL>(s, atoms, cpar, a, 0, [&](const Site& S) { return is_near(S, c, r1, zlo, zhi); },
+        total = collect<MODEL>(s, atoms, cpar, a, 0, [&](const Site& S) { return is_near<MODEL>(S, c, n1); },
                                [&](int n) {
                                    nfar += n;
                                    if (wave >= n) return;
@@ -477,7 +529,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
                 const Centre ct = centre_of(a, i0, j0, k0, kB - 0.5);
                 __syncthreads();
                 collect<MODEL>(s, atoms, cpar, a, r * kList,
-                               [&](const Site& S) { return !TWO || is_near(S, ct, r1, zlo, zhi); }, [](int) {});
+                               [&](const Site& S) { return !TWO || is_near<MODEL>(S, ct, n1); }, [](int) {});
             }
             return min(kList, total - r * kList);
         };
@@ -487,7 +539,7 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
             for (int i = 0; i < n; i += 256) {
                 const int e = i + (int)threadIdx.x;
                 const bool ok = e < n;
-                const bool nr = ok && is_near(s.list[e], c, r0, zlo, zhi);
+                const bool nr = ok && is_near<MODEL>(s.list[e], c, n0);
                 int rn, nn, rm, nm;
                 __syncthreads();
                 ranks(ok && nr, ok && !nr, s.cnt, rn, nn, rm, nm);

@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-from tests.test_gpu_grid_far import CASES, project, setup      # noqa: E402
+from oracle import oracle as O                                     # noqa: E402
+from tests.test_gpu_grid_far import CASES, project, setup, voxel_points      # noqa: E402
 
 
 @pytest.mark.parametrize("name", ["one_level_morse", "two_levels"])
@@ -23,3 +24,36 @@ def test_fp64_sums_do_not_depend_on_the_order_of_the_atoms(name):
     print(f"[acc64] {name}: {int(off.sum())} of {off.numel()} differ")
     assert off.float().mean() <= 1e-3
     assert (((a - b).abs() <= 2.0 ** -23 * a.abs() + 1e-12) | ~off).all()
+
+
+def heights(s, lo, hi, rng, k):
+    """k voxels (indices, flat and by axis) between lo and hi above the grid's z = 0."""
+    sp = s[2]
+    z = np.arange(sp.n[2]) * sp.dC[2] + sp.p0[2]
+    ok = np.nonzero((z >= lo) & (z < hi))[0]
+    i = np.stack([rng.integers(0, sp.n[0], k), rng.integers(0, sp.n[1], k), rng.choice(ok, k)], 1)
+    return (i[:, 2] * sp.n[1] + i[:, 1]) * sp.n[0] + i[:, 0], i
+
+
+def values(model, s, i, cp):
+    """FP64 field at voxels i (uncapped) of the pair parameters cp, at the FP32 positions of voxels and images."""
+    atoms, _, sp, Qs, QZs, npbc, lvA, lvB = s
+    f = np.float32
+    im = [(f(x), f(y)) for y in range(-npbc[1], npbc[1] + 1) for x in range(-npbc[0], npbc[0] + 1)]
+    sites = np.concatenate([np.c_[(atoms[:, :3] + x * lvA) + y * lvB, atoms[:, 3:]] for x, y in im]).astype(f)
+    return O.pair_fe(model, sites, np.tile(cp, (len(im), 1)), voxel_points(sp, i), Qs, QZs)
+
+
+@pytest.mark.parametrize("step,n", [(0.03, (260, 250, 200)), (0.04, (230, 220, 170))])
+def test_fine_lj_grids_without_charges(step, n):
+    """The r^-13 forces of atoms 10 half-widths (2.3 and 3 A) away.  Against FP64 at the FP32 positions, of the sum of
+    the repulsive and attractive fields: differences of positions below 8 A carry 2.4e-7 A, which enter 14 / r-fold
+    (1.2e-6 at 2.8 A), a reciprocal root of 1 ulp 14-fold (1.7e-6), the other roundings and the interpolation (kTol)
+    1e-6: 5e-6."""
+    s = setup(0, 60, 1, n, step, "none", 0.0)[:-2] + tuple(22.0 * np.eye(3, dtype=np.float32)[:2])
+    flat, i = heights(s, 2.2, 4.0, np.random.default_rng(2), 20000)
+    got = project(s, cap=False).cpu().numpy().reshape(-1, 4)[flat].astype(np.float64)
+    one = [values(0, s, i, (s[1] * np.array(m, np.float32))) for m in ((1, 0), (0, 1))]
+    err = np.abs(got - (one[0] + one[1])).max(1) / sum(np.linalg.norm(v, axis=1) for v in one)
+    print(f"[fine] {step}: largest {err.max():.1e}, rms {np.sqrt((err ** 2).mean()):.1e}")
+    assert err.max() <= 5e-6
