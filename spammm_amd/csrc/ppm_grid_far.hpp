@@ -134,9 +134,8 @@ __host__ __device__ inline double expected_near(const GridArgs& a, double r2) {
     return e < n ? e : n;
 }
 
-// The form of a whole grid: 0 the direct sum, 1 one level of blocks, 2 two levels (LJ only: over the
-// 3.1 A of 32 voxels the tail of a Morse exponential is not resolved by 8 nodes to the relative
-// accuracy of the direct sum).  It depends on the grid, never on the planes a launch stores, and is
+// The form of a whole grid: 0 the direct sum, 1 one level of blocks, 2 two levels (LJ only: 2 I_8(K h)
+// of 32 voxels is 300 times that of 16 or more).  It depends on the grid, never on the planes a launch stores, and is
 // plain double arithmetic, so host and device agree.
 // Costs are in pair evaluations, of which the card does 2.9e9 per ms (5.8e7: the 20 us any launch
 // takes): direct N per voxel; one level 512 N_far + 4096 N_near per block and 25e3 for its
@@ -147,8 +146,10 @@ __host__ __device__ inline double expected_near(const GridArgs& a, double r2) {
 // an eighth of the workgroups: measured, one level against two: 300x300x240 voxels with 60 sites 165 /
 // 253 us, 180 sites 253 / 225, 540 655 / 401, 1800 2114 / 722; 160^3 with 1800 538 / 596; 200x200x40
 // with 2304 320 / 357, with 5184 772 / 574.
+// A Morse field without tip charges is summed directly (is_near).
 __host__ __device__ inline int far_level(const GridArgs& a, int model) {
     if (a.dC[0] != 0.f || a.dC[1] != 0.f) return 0;
+    if (model == PPM_MODEL_MORSE && a.q0 == 0.f && a.noff == 0) return 0;
     const double n = (double)a.nsites, vox = (double)a.nx * a.ny * a.nz;
     const double near = expected_near(a, near2(a, model, false));
     const double per = 512.0 * (n - near) + 4096.0 * near;
@@ -209,6 +210,11 @@ __device__ __forceinline__ bool closer(const Site& S, const Centre& c, float r2,
 }
 
 // Near the centre c: closer than kRatio half-widths, or with an interpolation error above kTol of the site's terms.
+// Morse: the error of e^(-K r) is 2 I_8(K h) of its value at the centre, at any distance (2 (K h / 2)^8 / 8! and a
+// little more; taken twice: FP64 over a block's voxels gives up to 1.7 times it at K h <= 2).  It is weighed against the
+// charges' terms alone: a field of exponentials keeps the direct sum, whose error the interpolated one exceeds at every
+// K h >= 0.4 (rms 1.2 to 1.8 times at K = -1.8 and 0.03 to 0.1 A, 160 times at 0.2 A), so that atoms or tips without
+// charges are near at any distance.
 // LJ without charges, rms error against FP64 of the direct sum | with kRatio alone | so, relative, where kRatio alone is
 // worst: 0.04 A voxels at 3 A 9.5e-7 | 4.5e-6 | 2.7e-7, 0.03 A at 2 A 1.1e-6 | 2.5e-6 | 6.4e-7.
 template <int MODEL>
@@ -222,6 +228,17 @@ __device__ __forceinline__ bool is_near(const Site& S, const Centre& c, const Ne
         const float t6 = fabsf(S.c2) * i6, t12 = fabsf(S.c3) * i6 * i6;              // forces times distance
         const float tc = fabsf(S.q) * n.q * sqrtf(d2) / (dxy2 + fq * fq);
         return !(e4 * e4 * (kErr6 * t6 + kErr12 * t12) <= kTol * (t6 + t12 + tc));
+    }
+    if constexpr (MODEL == PPM_MODEL_MORSE) {
+        const float dx = S.x - c.x, dy = S.y - c.y, dz = S.z - c.z, dxy2 = dx * dx + dy * dy;
+        const float up = dz - n.zlo, lo = dz - n.zhi, fq = fmaxf(fabsf(up), fabsf(lo));
+        const float r = sqrtf(dxy2 + dz * dz), ex = gc::ex2(fmaf(S.c2, r, S.c0));
+        const float u = S.c2 * S.c2 * n.h2 * 0.480453f;                              // (K h)^2
+        auto err = [](float x2) { const float x4 = x2 * x2; return x4 * x4 * gc::ex2(0.04f * x2); };
+        // forces: the exponentials' errors, with what any field of this distance has (1e-8), against the charges
+        const float t = fabsf(S.c1) * ex * (fabsf(S.c3) + 1.0f / r);
+        const float tc = fabsf(S.q) * n.q / (dxy2 + fq * fq);
+        return !(t * (1e-8f + 3.9e-7f * (err(u) + ex * err(4.0f * u))) <= kTol * tc);
     }
     return false;
 }
@@ -281,6 +298,7 @@ __device__ __forceinline__ void add_site(const Site& S, const GridArgs& a, float
             f[k][3] += eo;
         }
     };
+    if (OFF == gc::kOffNone || S.q == 0.f) return;          // the same for the whole wave: S comes from LDS
     if constexpr (OFF == gc::kOffStatic) {
 #pragma unroll
         for (int o = 0; o < 4; ++o) {

@@ -57,3 +57,28 @@ def test_fine_lj_grids_without_charges(step, n):
     err = np.abs(got - (one[0] + one[1])).max(1) / sum(np.linalg.norm(v, axis=1) for v in one)
     print(f"[fine] {step}: largest {err.max():.1e}, rms {np.sqrt((err ** 2).mean()):.1e}")
     assert err.max() <= 5e-6
+
+
+@pytest.mark.parametrize("step,n,K,tip,charged,lo,hi", [
+    (0.2, (110, 110, 110), -1.8, "none", True, 12.0, 19.0),        # above the near radius of every atom
+    (0.125, (176, 176, 140), -1.8, "q0", False, 9.0, 15.0),        # a charged tip over atoms without charges
+    (0.04, (230, 220, 170), -2.5, "none", True, 2.5, 4.5),
+    (0.04, (230, 220, 170), -3.5, "q0", True, 2.5, 4.5),
+    (0.1, (130, 130, 120), -1.8, "offsets", True, 3.0, 10.0),      # charges of both signs, interpolated
+])
+def test_morse_exponents(step, n, K, tip, charged, lo, hi):
+    """Against FP64 at the FP32 positions, of the Morse field and (4e-6) of the charge terms: r carries 3 ulp at most, the
+    exponent K r 1.5e-5 up to K r = 45, the exponent's rounding 2.6e-6, the rest 1e-6: 2e-5."""
+    s = list(setup(1, 60, 1, n, step, tip, 0.0)[:-2] + tuple(22.0 * np.eye(3, dtype=np.float32)[:2]))
+    s[1][:, 2] = K
+    if not charged:
+        s[0][:, 3] = 0.0
+    flat, i = heights(s, lo, hi, np.random.default_rng(2), 6000)
+    got = project(tuple(s), cap=False).cpu().numpy().reshape(-1, 4)[flat].astype(np.float64)
+    want = values(1, s, i, s[1])
+    morse = np.linalg.norm(values(1, s[:3] + [[0] * 4] + s[4:], i, s[1]), axis=1)
+    P = voxel_points(s[2], i).astype(np.float64)
+    S = sum(O.abs_term_sums(s[0], np.zeros((60, 2)), q, s[5], s[6], s[7], P + [0, 0, z]) for q, z in zip(*s[3:5]) if q)
+    ratio = np.abs(got - want).max(1) / (2e-5 * morse + 4e-6 * S)
+    print(f"[morse] {step} {K} {tip}: largest error / bound {ratio.max():.2e}")
+    assert ratio.max() <= 1
