@@ -507,6 +507,13 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         for (int k = 0; k < kM; ++k) oz[k] = fmaf(a.dC[2], (float)kNode[k] * half, o);
     };
 
+    // sites first, first + 1, ... into the list: of one level every site passes through it (a look for them among all
+    // sites in each round made 180,000 Morse sites on 100x100x60 voxels take 291 ms; so 18.6, the direct sum 108)
+    auto load_sites = [&](int first) {
+        for (int i = threadIdx.x; i < kList && first + i < a.nsites; i += 256)
+            gc::load_site<MODEL>(atoms, cpar, a, first + i, s.list[i]);
+        __syncthreads();
+    };
     bool top = false;
     int total;
     if constexpr (TWO) {
@@ -532,7 +539,8 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         top = nfar > 0;
         if (top) reduce_nodes(s, f, s.top);
     } else {
-        total = collect<MODEL>(s, atoms, cpar, a, 0, [](const Site&) { return true; }, [](int) {});
+        total = a.nsites;
+        load_sites(0);
     }
     const int rounds = (total + kList - 1) / kList;
 
@@ -544,10 +552,14 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         const Centre c = centre_of(a, bi, bj, bk, 0.5 * (kB - 1));
         auto load_round = [&](int r) {              // the sites of this round into the list (one round: there)
             if (rounds > 1) {
-                const Centre ct = centre_of(a, i0, j0, k0, kB - 0.5);
                 __syncthreads();
-                collect<MODEL>(s, atoms, cpar, a, r * kList,
-                               [&](const Site& S) { return !TWO || is_near<MODEL>(S, ct, n1); }, [](int) {});
+                if constexpr (TWO) {
+                    const Centre ct = centre_of(a, i0, j0, k0, kB - 0.5);
+                    collect<MODEL>(s, atoms, cpar, a, r * kList,
+                                   [&](const Site& S) { return is_near<MODEL>(S, ct, n1); }, [](int) {});
+                } else {
+                    load_sites(r * kList);
+                }
             }
             return min(kList, total - r * kList);
         };

@@ -82,3 +82,23 @@ def test_morse_exponents(step, n, K, tip, charged, lo, hi):
     ratio = np.abs(got - want).max(1) / (2e-5 * morse + 4e-6 * S)
     print(f"[morse] {step} {K} {tip}: largest error / bound {ratio.max():.2e}")
     assert ratio.max() <= 1
+
+
+def test_time_of_one_level_grows_with_the_sites():
+    """Four times the sites take four times as long (and up to 1.4 times that), not sixteen."""
+    def ms(na):
+        s = list(setup(1, 8, 1, (96, 96, 48), 0.1, "q0", 0.0))
+        rng = np.random.default_rng(1)
+        s[0], s[1] = (np.repeat(v, na // 8, 0) for v in s[:2])
+        s[0][:, :2] = rng.uniform(-50, 50, (na, 2))
+        s[-2:] = 100.0 * np.eye(3, dtype=np.float32)[:2]
+        project(s)
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+        for e in t:
+            e.record()
+            project(s)
+        torch.cuda.synchronize()
+        return min(p.elapsed_time(q) for p, q in zip(t, t[1:]))
+    few, many = ms(4000), ms(16000)
+    print(f"[sites] 36,000 {few:.2f} ms, 144,000 {many:.2f} ms")
+    assert many <= 5.6 * few
