@@ -8,6 +8,7 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 from oracle import oracle as O                                     # noqa: E402
+from spammm_amd import device as D                                 # noqa: E402
 from tests.test_gpu_grid_far import CASES, project, setup, voxel_points      # noqa: E402
 
 
@@ -102,3 +103,57 @@ def test_time_of_one_level_grows_with_the_sites():
     few, many = ms(4000), ms(16000)
     print(f"[sites] 36,000 {few:.2f} ms, 144,000 {many:.2f} ms")
     assert many <= 5.6 * few
+
+
+def lj_gradient(atoms, cp, spec, Qs, QZs, cot, lv):
+    """d(sum of cot . (F, E)) / d(x, y, z, q, c6, c12) of 3 x 3 images in FP64, at the voxels' exact positions."""
+    k = (cot != 0).any(-1).nonzero()
+    ax = [torch.as_tensor(np.asarray(v, np.float64)[:3], device=cot.device) for v in (spec.p0, spec.dA, spec.dB, spec.dC)]
+    P = ax[0] + k[:, 2:] * ax[1] + k[:, 1:2] * ax[2] + k[:, :1] * ax[3]
+    g = cot[k[:, 0], k[:, 1], k[:, 2]].double()
+    f = np.float32
+    charges = [(float(f(q) * f(14.3996448915)), float(f(z))) for q, z in zip(Qs, QZs) if q]     # FP32 in the kernels too
+    out = []
+    for j in range(len(atoms)):
+        v = torch.cat([atoms[j], cp[j]]).double().requires_grad_(True)
+        tot = torch.zeros(6, dtype=torch.float64, device=cot.device)
+        for iy, ix in np.ndindex(3, 3):
+            d = P - v[:3] - torch.as_tensor((ix - 1.0) * lv[0] + (iy - 1.0) * lv[1], device=cot.device).double()
+            i2 = 1 / ((d * d).sum(1) + 1e-4)
+            gd = (g[:, :3] * d).sum(1)
+            L = ((v[5] * i2 ** 3 - v[4]) * i2 ** 3 * g[:, 3] + (12 * v[5] * i2 ** 3 - 6 * v[4]) * i2 ** 4 * gd).sum()
+            for q, zo in charges:
+                i1 = (d[:, 0] ** 2 + d[:, 1] ** 2 + (d[:, 2] + zo) ** 2 + 1e-4).rsqrt()
+                L = L + (q * v[3] * i1 * (g[:, 3] + i1 * i1 * (gd + zo * g[:, 2]))).sum()
+            tot += torch.autograd.grad(L, v)[0]
+        out.append(tot)
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("tip", ["q0", "offsets"])
+def test_interpolated_adjoint_is_no_further_off_than_the_direct_one(tip):
+    """A cotangent of one sign, 507 blocks of voxels at once (interpolated) and layer by layer (169 blocks: too few, direct).
+    The planes lie far up in the grid, where dC ic is large and the heights are not.  Per column, rms over the atoms against FP64: the near sites' roundings are the same in both, the rest is to be
+    smaller; 1.15 allows for chance in 60 to 180 values."""
+    n, step = (208, 208, 448), 0.05
+    atoms, cp, _, Qs, QZs, npbc, _, _ = setup(0, 60, 1, (8, 8, 8), step, tip, 0.0)
+    L = np.array(n) * step
+    spec = D.axis_aligned_spec([-L[0] / 2, -L[1] / 2, atoms[:, 2].max() - 17.0], L, n)
+    lv = 22.0 * np.eye(3, dtype=np.float32)[:2]
+    A, C = (torch.as_tensor(v, device=D.require_gpu()) for v in (atoms, cp))
+    cot = torch.zeros((n[2], n[1], n[0], 4), device=A.device)
+    rng = np.random.default_rng(8)
+    cot[400:440] = torch.as_tensor(1 + 0.2 * np.abs(rng.normal(size=(40, n[1], n[0], 4))).astype(np.float32))
+    grid = torch.zeros_like(cot)
+
+    def grad(c):
+        return D.grid_adjoint(A, C, 0, spec, Qs, QZs, grid, c, npbc, *lv, cap=True, params=True).to(A.device)
+    whole, direct = grad(cot), 0
+    for k in range(400, 448, 16):
+        part = torch.zeros_like(cot)
+        part[k:k + 16] = cot[k:k + 16]
+        direct = direct + grad(part)
+    want = lj_gradient(A, C, spec, Qs, QZs, cot, lv)
+    rms = [[float((g - want)[:, c].square().mean().sqrt()) for c in (slice(0, 3), 3, 4, 5)] for g in (whole, direct)]
+    print(f"[adjoint] {tip}: rms error interpolated / direct of xyz, q, c6, c12:", *(f"{a / b:.2f}" for a, b in zip(*rms)))
+    assert all(a != b for a, b in zip(*rms)) and all(a <= 1.15 * b for a, b in zip(*rms))
