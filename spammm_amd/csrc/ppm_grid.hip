@@ -417,11 +417,46 @@ __global__ __launch_bounds__(256) void k_grid_adjoint(const float4* __restrict__
 // form's positions (one FMA an axis) and, for q, whose near and far parts cancel, FINE in both parts.
 constexpr int kFarRows = 2048;      // workgroups (x shares) and rows of partials
 constexpr int kNearList = 512;
-// Near sites: closer than this many half-widths of a block (10 in the projection).  The terms are one derivative steeper
-// than the field: at 10, gradients on a 0.05 A grid were up to 5 times further off FP64 than the direct form's.
-constexpr double kAdjRatio = 12.5;
-inline double adj_near2(const GridArgs& a) {
-    return gf::half2(a, false) * kAdjRatio * kAdjRatio;
+// Near sites: closer than kAdjRatio half-widths of a block (10 in the projection: the terms are one derivative steeper
+// than the field), and farther out by the projection's rule (gf::is_near) for the derivatives r^-8 and r^-14 or of
+// exponentials against the charges'.
+constexpr float kAdjRatio = 12.5f;
+constexpr float kAdjErr6 = 50.3f, kAdjErr12 = 1590.f;       // C(p + 7, 8) / 2^7 of p = 8 and 14
+
+// PAR (LJ): the c12 column stands alone, and its r^-14 terms may be off by 4 kTol (13.3 half-widths).  The transposed sum
+// is a cotangent's product with the interpolation error, which alternates within a block.
+template <int MODEL, bool PAR>
+__device__ __forceinline__ bool adj_near(const float4& at, const gf::Centre& c, const gf::NearRule& n, float p0, float p1,
+                                         float K) {
+    gc::Site S{};
+    S.x = at.x; S.y = at.y; S.z = at.z;
+    if (gf::closer(S, c, kAdjRatio * kAdjRatio * n.h2, n.zlo, n.zhi)) return true;
+    const float dx = at.x - c.x, dy = at.y - c.y, dz = at.z - c.z, dxy2 = dx * dx + dy * dy, d2 = dxy2 + dz * dz;
+    const float fq = fmaxf(fabsf(dz - n.zlo), fabsf(dz - n.zhi)), q2 = dxy2 + fq * fq;
+    const float tc = 2.0f * fabsf(at.w) * n.q / (q2 * sqrtf(q2));
+    if constexpr (MODEL == PPM_MODEL_LJ) {
+        const float i2 = 1.0f / d2, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2, e8 = e4 * e4;
+        if (PAR && !(e8 * kAdjErr12 <= 4.0f * gf::kTol)) return true;
+        const float t6 = fabsf(42.f * p0) * i6, t12 = fabsf(156.f * p1) * i6 * i6;   // times distance squared
+        return !(e8 * (kAdjErr6 * t6 + kAdjErr12 * t12) <= gf::kTol * (t6 + t12 + tc * d2));
+    } else {
+        const float r = sqrtf(d2), ex = __expf(K * (r - p0)), t = fabsf(p1) * (2.0f * fabsf(K) + 1.0f / r) * (fabsf(K) + 1.0f / r);
+        return !(t * gf::morse_error(ex, K * K * n.h2) <= gf::kTol * tc);
+    }
+}
+
+// Squared near radius for the costs (an uncharged LJ atom as gf::near2's; Morse with charges: kAdjRatio).
+inline double adj_near2(const GridArgs& a, int model, bool params) {
+    const double h2 = gf::half2(a, false);
+    double q2 = (double)kAdjRatio * kAdjRatio;
+    if (model == PPM_MODEL_LJ) {
+        if (params) q2 = std::max(q2, 13.3 * 13.3);
+        for (int i = 0; i < 40; ++i, q2 *= 1.03) {
+            const double i2 = 12.25 / (q2 * h2), t12 = 156.0 / 84.0 * 2.0 * i2 * i2 * i2, w = 1.0 / (q2 * q2 * q2 * q2);
+            if (w * (kAdjErr6 + kAdjErr12 * t12) <= gf::kTol * (1.0 + t12)) break;
+        }
+    }
+    return q2 * h2;
 }
 
 struct AdjFar {
@@ -523,8 +558,7 @@ struct AdjShared {
 
 template <int MODEL, bool OFFS, bool PAR>
 __global__ __launch_bounds__(256, 3) void k_adj_far(const float4* __restrict__ atoms, const float* __restrict__ cpar,
-                                                    GridArgs a, AdjFar f, float near_r2, float zlo, float zhi,
-                                                    const float4* __restrict__ gcot, const int* __restrict__ list,
+                                                    GridArgs a, AdjFar f, const float4* __restrict__ gcot, const int* __restrict__ list,
                                                     const int* __restrict__ total, double* __restrict__ partials,
                                                     int* __restrict__ active) {
 #pragma clang fp contract(fast)
@@ -532,6 +566,7 @@ __global__ __launch_bounds__(256, 3) void k_adj_far(const float4* __restrict__ a
     constexpr int NC = PAR ? 6 : 4, cs = MODEL == PPM_MODEL_LJ ? 2 : 4;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n_list = *total, row = blockIdx.x;
+    const gf::NearRule rule = gf::near_rule<OFFS ? kOffStatic : kOffNone>(a, false);
     if (row >= n_list) {
         if (tid == 0 && blockIdx.y == 0) active[row] = 0;
         return;
@@ -659,9 +694,7 @@ __global__ __launch_bounds__(256, 3) void k_adj_far(const float4* __restrict__ a
             float4 at;
             float p0, p1, K;
             site(ok ? i : s_end - 1, at, p0, p1, K);
-            gc::Site S{};
-            S.x = at.x; S.y = at.y; S.z = at.z;
-            const bool nr = ok && gf::closer(S, c, near_r2, zlo, zhi);
+            const bool nr = ok && adj_near<MODEL, PAR>(at, c, rule, p0, p1, K);
             int rk, nk, ro, no;
             gf::ranks(nr, ok && !nr, s.cnt, rk, nk, ro, no);
             if (nr) s.list[n_near + rk] = i;
@@ -910,9 +943,11 @@ static AdjFar adj_far(const PpmGridSpec& g) {
 // with 9 % of the columns touched (1.1e9 evaluations direct) 0.89 | 0.61; 60 x 9 on 480 x 480 x 149 at 0.05 A 4.4 | 2.1,
 // on 150 x 150 x 120 at 0.1 A (8.8e8) 0.55 | 0.60; 200 on 180 x 180 x 120 0.51 | 0.52; 20 x 9 on 160 x 160 x 120
 // 0.26 | 0.57.  The first bound on the whole grid keeps small grids clear of the block kernels (30 us).
-static int adj_far_least(const GridArgs& a, const AdjFar& f) {
+static int adj_far_least(const GridArgs& a, const AdjFar& f, int model, bool params) {
     if (a.dC[0] != 0.f || a.dC[1] != 0.f) return 0;
-    const double n = a.nsites, near = gf::expected_near(a, adj_near2(a)), direct = 4096.0 * n;
+    // Morse: the parameters' columns are exponentials alone, and without tip charges every column is (gf::is_near)
+    if (model == PPM_MODEL_MORSE && (params || (a.q0 == 0.f && a.noff == 0))) return 0;
+    const double n = a.nsites, near = gf::expected_near(a, adj_near2(a, model, params)), direct = 4096.0 * n;
     const double far = 512.0 * 256.0 * std::ceil(n / 256.0) + 4096.0 * 64.0 * std::ceil(near / 64.0) + 40e3;
     if (far > 0.45 * direct || direct * f.bx * f.by * f.bz < 4e9) return 0;
     return std::max(1, (int)std::ceil(1e9 / direct));
@@ -978,7 +1013,7 @@ int launch_grid_adjoint(int model, const float* atoms, const float* cpar, int na
     if (V == 8) hipLaunchKernelGGL(k_adj_mark<8>, blocks, dim3(256), 0, stream, a, gc, w.flag, w.count);
     else hipLaunchKernelGGL(k_adj_mark<4>, blocks, dim3(256), 0, stream, a, gc, w.flag, w.count);
     const AdjFar far = adj_far(g);
-    if (const int least = adj_far_least(a, far)) {
+    if (const int least = adj_far_least(a, far, model, params)) {
         const int nblk = far.bx * far.by * far.bz;
         hipLaunchKernelGGL(k_adj_blocks, dim3((unsigned)nblk), dim3(256), 0, stream, a, far, G, gc, (int)blocks.x * 256, w.flag,
                            w.state);
@@ -986,18 +1021,14 @@ int launch_grid_adjoint(int model, const float* atoms, const float* cpar, int na
                            w.n_blocks);
         hipLaunchKernelGGL(k_adj_count, blocks, dim3(256), 0, stream, a, far, w.state, w.n_blocks, w.flag, w.count);
         if (int r = check_launch("grid_adjoint_blocks")) return r;
-        float zlo = 0.f, zhi = 0.f;
-        for (int o = 0; o < a.noff; ++o) { zlo = std::min(zlo, a.zoff[o]); zhi = std::max(zhi, a.zoff[o]); }
         const dim3 fb((unsigned)far.rows, (unsigned)std::max(1, std::min(4, na / 8)));
-        const float near_r2 = (float)adj_near2(a);
 #define PPM_ADJF(M, OF, PA) \
-    hipLaunchKernelGGL((k_adj_far<M, OF, PA>), fb, dim3(256), 0, stream, at, cpar, a, far, near_r2, zlo, zhi, gc, w.blocks, \
-                       w.n_blocks, partials + nb * (size_t)na * 6, active + nb)
-#define PPM_ADJF2(M) \
-    if (offs) { if (params) PPM_ADJF(M, true, true); else PPM_ADJF(M, true, false); } \
-    else { if (params) PPM_ADJF(M, false, true); else PPM_ADJF(M, false, false); }
-        if (model == PPM_MODEL_LJ) { PPM_ADJF2(PPM_MODEL_LJ) }
-        else { PPM_ADJF2(PPM_MODEL_MORSE) }
+    hipLaunchKernelGGL((k_adj_far<M, OF, PA>), fb, dim3(256), 0, stream, at, cpar, a, far, gc, w.blocks, w.n_blocks, \
+                       partials + nb * (size_t)na * 6, active + nb)
+#define PPM_ADJF2(M, PA) if (offs) PPM_ADJF(M, true, PA); else PPM_ADJF(M, false, PA)
+        if (model == PPM_MODEL_MORSE) { PPM_ADJF2(PPM_MODEL_MORSE, false); }
+        else if (params) { PPM_ADJF2(PPM_MODEL_LJ, true); }
+        else { PPM_ADJF2(PPM_MODEL_LJ, false); }
 #undef PPM_ADJF2
 #undef PPM_ADJF
         if (int r = check_launch("grid_adjoint_far")) return r;

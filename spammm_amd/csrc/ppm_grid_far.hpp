@@ -209,6 +209,12 @@ __device__ __forceinline__ bool closer(const Site& S, const Centre& c, float r2,
     return !(dx * dx + dy * dy + dz * dz >= r2);
 }
 
+// Interpolation error of ex (ex - 2), ex = e^(-K r) up to a factor, at (K h)^2 = u; 1e-8 is what the distance alone gives.
+__device__ __forceinline__ float morse_error(float ex, float u) {
+    auto bessel = [](float x2) { const float x4 = x2 * x2; return x4 * x4 * gc::ex2(0.04f * x2); };
+    return ex * (1e-8f + 3.9e-7f * (bessel(u) + ex * bessel(4.0f * u)));
+}
+
 // Near the centre c: closer than kRatio half-widths, or with an interpolation error above kTol of the site's terms.
 // Morse: the error of e^(-K r) is 2 I_8(K h) of its value at the centre, at any distance (2 (K h / 2)^8 / 8! and a
 // little more; taken twice: FP64 over a block's voxels gives up to 1.7 times it at K h <= 2).  It is weighed against the
@@ -233,12 +239,9 @@ __device__ __forceinline__ bool is_near(const Site& S, const Centre& c, const Ne
         const float dx = S.x - c.x, dy = S.y - c.y, dz = S.z - c.z, dxy2 = dx * dx + dy * dy;
         const float up = dz - n.zlo, lo = dz - n.zhi, fq = fmaxf(fabsf(up), fabsf(lo));
         const float r = sqrtf(dxy2 + dz * dz), ex = gc::ex2(fmaf(S.c2, r, S.c0));
-        const float u = S.c2 * S.c2 * n.h2 * 0.480453f;                              // (K h)^2
-        auto err = [](float x2) { const float x4 = x2 * x2; return x4 * x4 * gc::ex2(0.04f * x2); };
-        // forces: the exponentials' errors, with what any field of this distance has (1e-8), against the charges
-        const float t = fabsf(S.c1) * ex * (fabsf(S.c3) + 1.0f / r);
+        const float t = fabsf(S.c1) * (fabsf(S.c3) + 1.0f / r);                     // forces
         const float tc = fabsf(S.q) * n.q / (dxy2 + fq * fq);
-        return !(t * (1e-8f + 3.9e-7f * (err(u) + ex * err(4.0f * u))) <= kTol * tc);
+        return !(t * morse_error(ex, S.c2 * S.c2 * n.h2 * 0.480453f) <= kTol * tc);
     }
     return false;
 }
