@@ -238,15 +238,16 @@ __device__ __forceinline__ f3 rotMatT(f3 v, f3 a, f3 b, f3 c) {
                a.z * v.x + b.z * v.y + c.z * v.z);
 }
 // The operands of a relaxation's roots and quotients so far.  RN: they take the forms of ppm_rn.hpp, which
-// hold in the middle of the exponent range: r^2 in [2^-94, 2^60], v.v = 0 or in it, f.f + kF2SAFE <= 2^60,
-// the quotient of the two 0 or >= 2^-94.  out() tells whether one lay outside (a NaN does); the caller then
+// hold in the middle of the exponent range: r^2 in [2^-66, 2^60] (r above tipForce's least, 1e-10), v.v = 0 or in it,
+// f.f + kF2SAFE <= 2^60, the quotient of the two 0 or >= 2^-66 (one bound for all: another minimum for r^2 alone made
+// relaxStrokes 7 % slower, and v.v below it means |f| < 1e-9).  out() tells whether one lay outside (a NaN does); the caller then
 // relaxes the column again with RN = false, the IEEE forms, which have the same bits inside.  Two integer
 // minima and maxima of the bits a step and no branch: with a test and a branch in every step the short forms
 // saved nothing (relaxStrokes of 100 x 80 points and 31 heights: 0.62 ms with the IEEE forms, 0.62 with the
 // branch, 0.55 as this).
 template <bool RN>
 struct MidRange {
-    static constexpr unsigned kLo = 0x10800000u, kHi = 0x5d800000u;      // bits of 2^-94 and 2^60
+    static constexpr unsigned kLo = 0x1e800000u, kHi = 0x5d800000u;      // bits of 2^-66 and 2^60
     unsigned lo = ~0u, hi = 0u;
     __device__ __forceinline__ void root(float rr) {
         if (RN) {

@@ -80,3 +80,24 @@ def test_direct_sum_bits_do_not_depend_on_the_lanes(n_many, n_few, na):
     n = n_few * n_few
     for many, few in zip(scan(n_many * n_many), scan(n)):
         assert torch.isfinite(many).all() and torch.equal(many[:n], few)
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4])
+def test_probe_within_1e_10_of_the_anchor(lanes):
+    """A probe that its first step takes to 2^-35 A (3e-11) from the anchor: the spring's length is 1e-10 there, in the
+    short forms as in IEEE's.  dt = 1/2 and a constant force of 4 (2^-35 - 2^-28) from the rest position 2^-28, where
+    the radial spring is at rest."""
+    n = (8, 8, 8)
+    sp = D.axis_aligned_spec([-2, -2, -2], [4, 4, 4], n)
+    g = np.zeros(n + (4,), np.float32)
+    g[..., 0] = 4 * (2.0 ** -35 - 2.0 ** -28)
+    tip = D.Tip(stiffness=np.array([0, 0, 0, -1], np.float32), dpos0=np.array([2.0 ** -28, 0, 0, 2.0 ** -28], np.float32),
+                relax=np.array([0.5, 0.1, 0.05, 0.5], np.float32), tipC=np.array([0, 0, 1, -0.125], np.float32))
+    pts = np.zeros((5, 4), np.float32)
+    G, P = (torch.as_tensor(v, device=dev()) for v in (g, pts))
+    for cb in (True, False):
+        FEs, PPs = D.relax_tilted(G, sp, P, 3, tip, 4, 1e-30, check_before=cb, lanes=lanes)
+        FEo, PPo = O.relax_tilted(g, sp.n, sp.dinvA, sp.dinvB, sp.dinvC, pts, 3, tip.tipA, tip.tipB, tip.tipC,
+                                  tip.stiffness, tip.dpos0, tip.relax, tip.surfFF, 4, 1e-30, cb, "f32")
+        np.testing.assert_array_equal(PPs.cpu().numpy(), PPo)
+        np.testing.assert_array_equal(FEs.cpu().numpy(), FEo)
