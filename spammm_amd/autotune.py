@@ -1,30 +1,32 @@
 """Autotuner of the batched forward's launch shape.
 
-Candidates: grid voxels per thread along z (4, 8), the pixel tile of a wavefront (16x4, 8x8,
-4x16 pixels), persistent workgroups per compute unit (2, 3, 4), the schedule (one library call,
-or one for the grid launch and one for the relaxation launch) and the queue order (lag 0: each
-molecule's relaxation blocks right after its tiles; k: after the tiles of molecule m + k).  Each candidate runs the real batch
-(or a prefix of it) and is timed with HIP events on the launch stream; every candidate's df
-must equal the first candidate's bit for bit (they compute the same arithmetic, only the
-work decomposition differs).  The winner is cached in a JSON file keyed by device name and a
-signature of the batch (number of molecules, pixels, z-steps, projected pair evaluations).
+Candidates: the size of a grid tile (4, 8), the pixel tile of a wavefront (16x4, 8x8, 4x16 pixels) and
+persistent workgroups per compute unit (2, 3, 4).  The schedule (one library call, or one for the grid
+launch and one for the relaxation launch) and the queue order (lag) only order items that the other
+launch passes over: a caller's candidates may name them, the default ones do not.  Each candidate runs
+the real batch (or a prefix of it) and is timed with HIP events on the launch stream; every candidate's
+df must equal the first candidate's bit for bit (they compute the same arithmetic, only the work
+decomposition differs).  The winner is cached in a JSON file keyed by the device's name, the library's
+build and a signature of the batch (number of molecules, pixels, z-steps, projected pair evaluations,
+model and tip charges): another build's kernels want other shapes.
 
 Cache file: $SPAMMM_AMD_TUNE_CACHE or ~/.cache/spammm_amd/autotune.json.
 """
 from __future__ import annotations
 
+import functools
+import hashlib
 import itertools
 import json
 import os
 
+from . import _lib
 from .batch import BatchForward, LaunchConfig
 
 CANDIDATES = {
     "vz": (4, 8),
     "tile_w": (4, 8, 16),
     "workers_per_cu": (2, 3, 4),
-    "schedule": ("fused", "two_phase"),
-    "lag": (0, 2, 8),
 }
 
 
@@ -35,11 +37,20 @@ def cache_path() -> str:
     return os.path.join(os.path.expanduser("~"), ".cache", "spammm_amd", "autotune.json")
 
 
+@functools.lru_cache(maxsize=None)
+def _build(path: str) -> str:
+    """Digest of the library file (read once per process: the library is loaded once)."""
+    with open(path, "rb") as f:
+        return hashlib.sha256(f.read()).hexdigest()[:12]
+
+
 def signature(batch: BatchForward) -> str:
     import torch
     name = torch.cuda.get_device_properties(batch.device).name
     pairs = batch.pair_evals
-    return f"{name}|nmol{len(batch.molecules)}|pix{batch.n_pix}|nz{batch.nz}|pairs{pairs:.3e}"
+    tip = "".join("-" if q == 0 else "0" if z == 0 else "z" for q, z in zip(batch.Qs, batch.QZs))
+    return (f"{name}|build{_build(_lib.LIB_PATH)}|nmol{len(batch.molecules)}|pix{batch.n_pix}|nz{batch.nz}"
+            f"|pairs{pairs:.3e}|model{batch.model}|tip{tip}")
 
 
 def _load():
@@ -114,11 +125,10 @@ def tune(batch: BatchForward, candidates=None, reps: int = 2, use_cache: bool = 
     return best, results
 
 
-def refine(batch: BatchForward, cfg: LaunchConfig, lags=(32, 64), reps: int = 2, log=None):
+def refine(batch: BatchForward, cfg: LaunchConfig, lags=(), reps: int = 2, log=None):
     """The tuned shape ``cfg`` checked on the whole ``batch``: the same vz, tile and workgroups per
-    CU as two-phase and as fused with each queue lag in ``lags`` (lags longer than the tuning
-    sample's molecule count), each timed on the whole batch; returns (the fastest, {key: ms}).  Every variant must give the first
-    one's results bit for bit."""
+    CU in two library calls and in one with each queue lag in ``lags``, each timed on the whole batch;
+    returns (the fastest, {key: ms}).  Every variant must give the first one's results bit for bit."""
     import torch
     variants = [cfg, LaunchConfig(cfg.vz, cfg.tile_w, cfg.workers_per_cu, "two_phase", 0)]
     variants += [LaunchConfig(cfg.vz, cfg.tile_w, cfg.workers_per_cu, "fused", int(lag)) for lag in lags

@@ -190,8 +190,8 @@ class BatchForward:
 
     def _set_items(self, cfg: LaunchConfig):
         """Work items of every molecule and the queue order of their segments: the grid tiles of
-        molecule m, then (lag = k) the relaxation blocks of molecule m - k, so that a block of m is
-        dequeued k molecules' tiles after the last tile of m (it rarely waits)."""
+        molecule m, then (lag = k) the relaxation blocks of molecule m - k.  The grid launch passes over
+        the blocks and the relaxation launch over the tiles, so the order between the kinds is free."""
         key = (cfg.vz, cfg.tile_w, cfg.lag)
         if self._items_for == key:
             return
@@ -314,7 +314,7 @@ class BatchForward:
             self.launch(cfg)
         err, flags = self.status()
         if err:
-            raise RuntimeError("batched forward: a relaxation block timed out waiting for its grid")
+            raise RuntimeError("batched forward: a molecule was relaxed before all its grid tiles were projected")
         bad = np.flatnonzero(flags)
         if bad.size:
             self.recompute_plain(bad)
