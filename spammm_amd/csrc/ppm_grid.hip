@@ -432,15 +432,15 @@ __device__ __forceinline__ bool adj_near(const float4& at, const gf::Centre& c, 
     S.x = at.x; S.y = at.y; S.z = at.z;
     if (gf::closer(S, c, kAdjRatio * kAdjRatio * n.h2, n.zlo, n.zhi)) return true;
     const float dx = at.x - c.x, dy = at.y - c.y, dz = at.z - c.z, dxy2 = dx * dx + dy * dy, d2 = dxy2 + dz * dz;
-    const float fq = fmaxf(fabsf(dz - n.zlo), fabsf(dz - n.zhi)), q2 = dxy2 + fq * fq;
-    const float tc = 2.0f * fabsf(at.w) * n.q / (q2 * sqrtf(q2));
+    const float fq = fmaxf(fabsf(dz - n.zlo), fabsf(dz - n.zhi)), iq = rsq(dxy2 + fq * fq), ir = rsq(d2);
+    const float tc = 2.0f * fabsf(at.w) * n.q * (iq * iq * iq);
     if constexpr (MODEL == PPM_MODEL_LJ) {
-        const float i2 = 1.0f / d2, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2, e8 = e4 * e4;
+        const float i2 = ir * ir, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2, e8 = e4 * e4;
         if (PAR && !(e8 * kAdjErr12 <= 4.0f * gf::kTol)) return true;
         const float t6 = fabsf(42.f * p0) * i6, t12 = fabsf(156.f * p1) * i6 * i6;   // times distance squared
         return !(e8 * (kAdjErr6 * t6 + kAdjErr12 * t12) <= gf::kTol * (t6 + t12 + tc * d2));
     } else {
-        const float r = sqrtf(d2), ex = __expf(K * (r - p0)), t = fabsf(p1) * (2.0f * fabsf(K) + 1.0f / r) * (fabsf(K) + 1.0f / r);
+        const float ex = __expf(K * (d2 * ir - p0)), t = fabsf(p1) * (2.0f * fabsf(K) + ir) * (fabsf(K) + ir);
         return !(t * gf::morse_error(ex, K * K * n.h2) <= gf::kTol * tc);
     }
 }

@@ -229,18 +229,20 @@ __device__ __forceinline__ bool is_near(const Site& S, const Centre& c, const Ne
     if constexpr (MODEL == PPM_MODEL_LJ) {
         const float dx = S.x - c.x, dy = S.y - c.y, dz = S.z - c.z, dxy2 = dx * dx + dy * dy;
         const float up = dz - n.zlo, lo = dz - n.zhi;
-        const float d2 = dxy2 + dz * dz, i2 = 1.0f / d2, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2;
-        const float fq = fmaxf(fabsf(up), fabsf(lo));            // the farthest charge
+        const float d2 = dxy2 + dz * dz;
+        if (d2 >= 256.f * n.h2) return false;                    // kErr12 (h/d)^8 < kTol
+        const float ir = gc::rsq(d2), i2 = ir * ir, i6 = i2 * i2 * i2, e2 = n.h2 * i2, e4 = e2 * e2;
+        const float fq = fmaxf(fabsf(up), fabsf(lo)), iq = gc::rsq(dxy2 + fq * fq);  // of the farthest charge
         const float t6 = fabsf(S.c2) * i6, t12 = fabsf(S.c3) * i6 * i6;              // forces times distance
-        const float tc = fabsf(S.q) * n.q * sqrtf(d2) / (dxy2 + fq * fq);
+        const float tc = fabsf(S.q) * n.q * (d2 * ir) * (iq * iq);
         return !(e4 * e4 * (kErr6 * t6 + kErr12 * t12) <= kTol * (t6 + t12 + tc));
     }
     if constexpr (MODEL == PPM_MODEL_MORSE) {
         const float dx = S.x - c.x, dy = S.y - c.y, dz = S.z - c.z, dxy2 = dx * dx + dy * dy;
-        const float up = dz - n.zlo, lo = dz - n.zhi, fq = fmaxf(fabsf(up), fabsf(lo));
-        const float r = sqrtf(dxy2 + dz * dz), ex = gc::ex2(fmaf(S.c2, r, S.c0));
-        const float t = fabsf(S.c1) * (fabsf(S.c3) + 1.0f / r);                     // forces
-        const float tc = fabsf(S.q) * n.q / (dxy2 + fq * fq);
+        const float up = dz - n.zlo, lo = dz - n.zhi, fq = fmaxf(fabsf(up), fabsf(lo)), iq = gc::rsq(dxy2 + fq * fq);
+        const float d2 = dxy2 + dz * dz, ir = gc::rsq(d2), ex = gc::ex2(fmaf(S.c2, d2 * ir, S.c0));
+        const float t = fabsf(S.c1) * (fabsf(S.c3) + ir);                           // forces
+        const float tc = fabsf(S.q) * n.q * (iq * iq);
         return !(t * morse_error(ex, S.c2 * S.c2 * n.h2 * 0.480453f) <= kTol * tc);
     }
     return false;
