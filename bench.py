@@ -197,7 +197,7 @@ def main():
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",
             "frac": grid_gbs / PEAK_HBM_GBS,
-            "traffic": w.nvox * 16.0,
+            "traffic": _pmc_traffic("k_grid_far", w.name),
             "work_unit": f"{w.nvox} voxels x 16 B written per launch",
             "all_pairs": pairs,
             "avg_launch_ms": p_grid,

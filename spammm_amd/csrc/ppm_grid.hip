@@ -11,7 +11,7 @@
 //
 // Two forms, chosen by far_level from the grid alone.  Grids of more than a few sites and blocks
 // take the interpolated one (ppm_grid_far.hpp): the flake's 300x300x240 voxels x 1800 sites 13.06 -> 0.73 ms,
-// a 9216-site slab on 320x320x96 at 0.05 A 32.9 -> 1.07 ms.  The rest is the direct sum (FP32 VALU-bound):
+// a 9216-site slab on 320x320x96 at 0.05 A 32.9 -> 1.04 ms.  The rest is the direct sum (FP32 VALU-bound):
 //   * one workgroup = 256 columns (ia,ib) x V consecutive z voxels per thread (V = 16 or 8
 //     for LJ, chosen per launch shape; 8 for Morse, 4 for a tilted dC, 1 for launches of few
 //     workgroups); voxels of one thread
@@ -942,7 +942,8 @@ static AdjFar adj_far(const PpmGridSpec& g) {
 // Milliseconds direct | interpolated with 45 planes touched: 200 atoms x 9 images on 300 x 300 x 240 voxels 6.5 | 2.0,
 // with 9 % of the columns touched (1.1e9 evaluations direct) 0.89 | 0.61; 60 x 9 on 480 x 480 x 149 at 0.05 A 4.4 | 2.1,
 // on 150 x 150 x 120 at 0.1 A (8.8e8) 0.55 | 0.60; 200 on 180 x 180 x 120 0.51 | 0.52; 20 x 9 on 160 x 160 x 120
-// 0.26 | 0.57.  The first bound on the whole grid keeps small grids clear of the block kernels (30 us).
+// 0.26 | 0.57 (k_adj_far takes 10 % more since its roots are finer).  The first bound on the whole grid keeps small
+// grids clear of the block kernels (30 us).
 static int adj_far_least(const GridArgs& a, const AdjFar& f, int model, bool params) {
     if (a.dC[0] != 0.f || a.dC[1] != 0.f) return 0;
     // Morse: the parameters' columns are exponentials alone, and without tip charges every column is (gf::is_near)

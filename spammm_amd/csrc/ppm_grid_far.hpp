@@ -646,7 +646,8 @@ __device__ __forceinline__ void far_blocks(Shared& s, const float4* __restrict__
         if (bi + x < a.nx && bj + y < a.ny) {
             const int col = (bj + y) * a.nx + bi + x;
             // base may be out: the compiler keeps a load behind the stores before it, so eight planes of base are
-            // read before the first of them is stored (480x480x149 with a base: 629 -> 522 us)
+            // read before the first of them is stored (480x480x149 with a base: 629 -> 522 us,
+            // 543 since the near set follows the error bound)
 #pragma unroll
             for (int k0 = 0; k0 < kB; k0 += kBase) {
                 float4 b[kBase];

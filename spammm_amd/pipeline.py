@@ -50,9 +50,10 @@ class ScanPipeline:
     tip: device.Tip; model: _lib.PPM_MODEL_LJ or _lib.PPM_MODEL_MORSE; Qs, QZs, npbc, lvA, lvB, cap:
     as device.grid_project; max_iter, f2conv, check_before, scan_ny, damped: as device.relax_tilted;
     df_op: a df.AxisOperator over nz slices (or None: no df); depth: buffer sets and streams (>= 2);
-    lanes: lanes per scan point of the relaxation (default 1: beside a grid projection the
-    relaxation's latency is hidden and only its instruction count matters, and one lane per point
-    issues the fewest; 0 = the library's choice for a launch alone on the GPU).
+    lanes: lanes per scan point of the relaxation (default 1: one lane per point issues the fewest
+    instructions, and its latency is hidden by the other stream's kernels: 200 atoms, 300x300x240 voxels and
+    256x256x60 steps take 2.48 ms per image with 1 lane, 2.83 with 2 and 3.84 with 4; 0 = the library's choice
+    for a launch alone on the GPU, 2 there).
     """
 
     def __init__(self, spec, points, nz, tip, model=_lib.PPM_MODEL_LJ, Qs=(0, 0, 0, 0), QZs=(0, 0, 0, 0),

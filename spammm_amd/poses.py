@@ -84,8 +84,9 @@ class Scene:
     # recomputed there)
     batch_depth: int = 2
     batch_grid_budget: float = 64 * 2 ** 30
-    # lanes per scan point of the batch's relaxations (device.relax_ctl): 1, the fewest instructions,
-    # since they run beside another placement's grid projection (0: the choice for a lone launch)
+    # lanes per scan point of the batch's relaxations (device.relax_ctl): 1, the fewest instructions, since
+    # they run beside another placement's kernels (0: the choice for a lone launch).  192x192x60 steps over a
+    # 480x480x149 window: 95 placements/s with 1 lane, 98 with 2, 96 with 0
     batch_lanes: int = 1
     batch_slots: list = field(default=None, repr=False)
 
